@@ -44,16 +44,52 @@ SR_HD uint32_t mmul(uint32_t a, uint32_t b) {
     uint32_t r = (uint32_t)(x & P) + (uint32_t)(x >> 31);
     return umin32(r, r - P);
 }
-// b * t mod p for canonical b, t given t2 = 2t (a plain u32): b*t2 = 2bt splits as
-// hi = floor(bt / 2^31) and lo / 2 = bt mod 2^31, so bt = hi + (lo >> 1) (mod p) with
-// hi + (lo >> 1) < 2p; one conditional subtraction canonicalises.
-SR_HD uint32_t mmul_t2(uint32_t b, uint32_t t2) {
-    uint64_t x = (uint64_t)b * t2;
-    uint32_t r = (uint32_t)(x >> 32) + ((uint32_t)x >> 1);
+// ---- butterflies on signed words (circle FFT) ----
+// A twiddle t is held as mtw2(t) = 2t or 2(t - p), whichever lies in (-p, p): for signed b the
+// 64-bit S = b mtw2(t) has S / 2 = b t (mod p).  With S = hi 2^32 + lo, rounded so that lo is in
+// [-2^31, 2^31), S / 2 = hi 2^31 + lo / 2 = hi + lo / 2 (mod p), and lo is even: a 62-bit S folds
+// to one signed word with a shift and an addition.  An addend folded into the multiply-add
+// does the rounding and keeps both terms in unsigned range, so the fold is mhalf(S + addend).
+SR_HD int32_t mtw2(uint32_t t) { return (int32_t)(2u * t - (t > P / 2 ? 2u * P : 0u)); }
+SR_HD uint32_t mhalf(int64_t s) { return (uint32_t)((uint64_t)s >> 32) + ((uint32_t)s >> 1); }
+// Forward butterfly (a, b) <- (a + b t, a - b t), 7 instructions: the sums S = 2a +- b mtw2(t) fold
+// directly.  |a|, |b| <= p give |S| <= 2^31 (p - 1) + 2^32 - 2 < 2^62, so hi is in
+// (-2^30, 2^30], lo / 2 in [-2^30, 2^30), and the results are in [-p, p - 1] again (hi = 2^30
+// only with lo < 0): no reduction between stages.  The addend 2^31 - 2^62 rounds and takes the
+// 2^30 that the unsigned lo >> 1 adds back off hi.
+SR_HD void mbfly(uint32_t& a, uint32_t& b, int32_t t2, int32_t neg_t2) {
+    constexpr int64_t K = 0x80000000ll - (1ll << 62);
+#ifdef __HIP_DEVICE_COMPILE__
+    int64_t s;  // one multiply-add; the compiler would take a shift and a 64-bit addition
+    asm("v_mad_i64_i32 %0, vcc, %1, 2, %2" : "=v"(s) : "v"(a), "s"(K) : "vcc");
+#else
+    const int64_t s = (int64_t)(int32_t)a * 2 + K;
+#endif
+    const int64_t x = (int64_t)(int32_t)b * t2 + s, y = (int64_t)(int32_t)b * neg_t2 + s;
+    a = mhalf(x);
+    b = mhalf(y);
+}
+// Canonical word of a signed word in [-p, p - 1].
+SR_HD uint32_t mcanon(uint32_t a) { return umin32(a, a + P); }
+// d t mod p in [0, p - 1] for a signed d in [-p, p]: |d mtw2(t)| <= p (p - 1) folds to
+// [-p, p - 1], the addend 2^31 + (2^30 - 1) 2^32 rounds and shifts it to [0, 2p - 1].
+SR_HD uint32_t mmul_s(uint32_t d, int32_t t2) {
+    const uint32_t r = mhalf((int64_t)(int32_t)d * t2 + (0x80000000ll + ((int64_t)((1 << 30) - 1) << 32)));
     return umin32(r, r - P);
 }
-// 2 * (p - w) for a doubled word w2 = 2w: the doubled negation (0 stays 0).
-SR_HD uint32_t mneg_t2(uint32_t w2) { return w2 == 0 ? 0u : 0xFFFFFFFEu - w2; }
+// Inverse butterfly (a, b) <- (a + b, (a - b) t) on words in [0, p]: the difference goes into
+// the product as it is (9 instructions).
+SR_HD void mibfly(uint32_t& a, uint32_t& b, int32_t t2) {
+    const uint32_t s = a + b;
+    b = mmul_s(a - b, t2);
+    a = umin32(s, s - P);
+}
+// The same times a scale: s2 = mtw2(scale), ts2 = mtw2(t scale); a + b enters as a + b - p.
+SR_HD void mibfly_scaled(uint32_t& a, uint32_t& b, int32_t s2, int32_t ts2) {
+    const uint32_t s = a + b - P;
+    b = mmul_s(a - b, ts2);
+    a = mmul_s(s, s2);
+}
 // Fold a 64-bit accumulator of folded products to a canonical word (m31.zig:150-158).
 SR_HD uint32_t mred64(uint64_t x) {
     uint64_t t = (x & P) + (x >> 31);

@@ -121,7 +121,11 @@ __global__ __launch_bounds__(FFT_THREADS) void fft_pass_kernel(const uint32_t* c
 // then the tile is exchanged through LDS so that the next 4 row bits become
 // thread-local: ceil(R/4) LDS exchanges per pass instead of R barriers.  R and
 // LOGC are template parameters, so the row mapping, strides and twiddle
-// offsets of every group are compile-time shifts.  Twiddles of one stage are
+// offsets of every group are compile-time shifts.  The passes are bound by their VALU
+// instructions and by HBM at about the same level (a 2^20 x 100 unit moves 4.2 GB), so the
+// butterflies work on words that no stage reduces: 7 instructions forward and 9 inverse
+// (fields.hpp) where canonical words took 11; the wide-Fibonacci 2^20 x 100 proof went from
+// 3.28 to 3.10 ms.  Twiddles of one stage are
 // consecutive tower words (one base + constant offsets).  The first group
 // loads from HBM, the last one stores to HBM.
 constexpr int RX_LOG = 4;  // 16 elements per thread
@@ -131,7 +135,8 @@ struct RxPass {
     uint32_t m, src_log;
     uint32_t s_lo;       // first stage of the pass
     uint32_t tower_log;
-    uint32_t scale;      // multiply on store when != 1 (last inverse pass)
+    uint32_t scaled;     // last inverse pass: its top stage multiplies by 2^-m
+    int32_t scale, scale_t;  // mtw2 of 2^-m and of 2^-m times the top stage's only twiddle
     uint32_t dup_top;    // forward: top stage pairs with zero padding (v1 = 0)
 };
 
@@ -178,7 +183,7 @@ __device__ __forceinline__ void rx_lds_get(uint32_t (&v)[RX], const uint32_t* ld
     }
 }
 
-// Twiddles of one stage (doubled tower words): RX >> (Q+1) consecutive words of T_{s-1}
+// Twiddles of one stage (signed doubled tower words, mtw2): RX >> (Q+1) consecutive words of T_{s-1}
 // for a line stage; for the circle stage the two (x, y) pairs of T_0 the thread needs.
 template <bool INV, int R, int LOGC, int B, int Q>
 __device__ __forceinline__ void rx_tw_load(uint32_t (&w)[8], const uint32_t* __restrict__ tower, const RxPass& ps,
@@ -203,52 +208,47 @@ __device__ __forceinline__ void rx_tw_load(uint32_t (&w)[8], const uint32_t* __r
     }
 }
 
-template <bool INV, int R, int LOGC, int B, int Q>
+// One stage on the thread's 16 values.  Forward values are signed words in [-p, p - 1] that no
+// stage reduces (mbfly); inverse values lie in [0, p].  SCALED: the top stage of the last
+// inverse pass (one twiddle for the whole transform) also multiplies by 2^-m.
+template <bool INV, int R, int LOGC, int B, int Q, bool SCALED>
 __device__ __forceinline__ void rx_stage(uint32_t (&v)[RX], const uint32_t (&w)[8], const RxPass& ps, bool dup) {
     constexpr int LS = B + Q;
     constexpr bool IS_CIRCLE = (LS == 0 && LOGC == 0);  // as in rx_tw_load
     if constexpr (!IS_CIRCLE) {
 #pragma unroll
         for (int hk = 0; hk < (RX >> (Q + 1)); hk++) {
-            const uint32_t tw = w[hk];
+            const int32_t tw = (int32_t)w[hk], ntw = -tw;
 #pragma unroll
             for (int lk = 0; lk < (1 << Q); lk++) {
                 const int k0 = (hk << (Q + 1)) | lk, k1 = k0 | (1 << Q);
-                uint32_t a = v[k0], c = v[k1];
                 if (!INV) {
-                    if (dup) {
-                        v[k1] = a;  // zero-padded partner: (a + 0*t, a - 0*t)
-                    } else {
-                        uint32_t tmp = mmul_t2(c, tw);
-                        v[k0] = madd(a, tmp);
-                        v[k1] = msub(a, tmp);
-                    }
+                    if (dup)
+                        v[k1] = v[k0];  // zero-padded partner: (a + 0*t, a - 0*t)
+                    else
+                        mbfly(v[k0], v[k1], tw, ntw);
+                } else if (SCALED && LS == R - 1) {
+                    mibfly_scaled(v[k0], v[k1], ps.scale, ps.scale_t);
                 } else {
-                    v[k0] = madd(a, c);
-                    v[k1] = mmul_t2(msub(a, c), tw);
+                    mibfly(v[k0], v[k1], tw);
                 }
             }
         }
     } else {
         // Circle stage (B == 0, Q == 0, s_lo == 0): pairs (2h', 2h'+1), h' = hp0 + hk,
         // twiddles [y, -y, -x, x] from consecutive pairs (x, y) of T_0.
-        const uint32_t x0 = w[0], y0 = w[1], x1 = w[2], y1 = w[3];
+        const int32_t x0 = (int32_t)w[0], y0 = (int32_t)w[1], x1 = (int32_t)w[2], y1 = (int32_t)w[3];
 #pragma unroll
         for (int hk = 0; hk < RX / 2; hk++) {
             const int k0 = 2 * hk, k1 = k0 + 1;
-            const uint32_t x = hk < 4 ? x0 : x1, y = hk < 4 ? y0 : y1;
+            const int32_t x = hk < 4 ? x0 : x1, y = hk < 4 ? y0 : y1;
             const int rr = hk & 3;
-            const uint32_t wv = rr < 2 ? y : x;
-            const uint32_t t = (rr == 1 || rr == 2) ? mneg_t2(wv) : wv;  // doubled words
-            uint32_t a = v[k0], c = v[k1];
-            if (!INV) {
-                uint32_t tmp = mmul_t2(c, t);
-                v[k0] = madd(a, tmp);
-                v[k1] = msub(a, tmp);
-            } else {
-                v[k0] = madd(a, c);
-                v[k1] = mmul_t2(msub(a, c), t);
-            }
+            const int32_t wv = rr < 2 ? y : x;
+            const bool neg = rr == 1 || rr == 2;
+            if (!INV)
+                mbfly(v[k0], v[k1], neg ? -wv : wv, neg ? wv : -wv);
+            else
+                mibfly(v[k0], v[k1], neg ? -wv : wv);
         }
     }
 }
@@ -264,18 +264,18 @@ __device__ __forceinline__ void rx_group_tw(uint32_t (&w)[4][8], const uint32_t*
     if (B + 0 >= LO && B + 0 < HI) rx_tw_load<INV, R, LOGC, B, 0>(w[0], tower, ps, hi, r, base);
 }
 
-template <bool INV, int R, int LOGC, int B, int LO, int HI>
+template <bool INV, int R, int LOGC, int B, int LO, int HI, bool SCALED>
 __device__ __forceinline__ void rx_group(uint32_t (&v)[RX], const uint32_t (&w)[4][8], const RxPass& ps, bool dup) {
     if (!INV) {
-        if (B + 3 >= LO && B + 3 < HI) rx_stage<INV, R, LOGC, B, 3>(v, w[3], ps, dup);
-        if (B + 2 >= LO && B + 2 < HI) rx_stage<INV, R, LOGC, B, 2>(v, w[2], ps, false);
-        if (B + 1 >= LO && B + 1 < HI) rx_stage<INV, R, LOGC, B, 1>(v, w[1], ps, false);
-        if (B + 0 >= LO && B + 0 < HI) rx_stage<INV, R, LOGC, B, 0>(v, w[0], ps, false);
+        if (B + 3 >= LO && B + 3 < HI) rx_stage<INV, R, LOGC, B, 3, SCALED>(v, w[3], ps, dup);
+        if (B + 2 >= LO && B + 2 < HI) rx_stage<INV, R, LOGC, B, 2, SCALED>(v, w[2], ps, false);
+        if (B + 1 >= LO && B + 1 < HI) rx_stage<INV, R, LOGC, B, 1, SCALED>(v, w[1], ps, false);
+        if (B + 0 >= LO && B + 0 < HI) rx_stage<INV, R, LOGC, B, 0, SCALED>(v, w[0], ps, false);
     } else {
-        if (B + 0 >= LO && B + 0 < HI) rx_stage<INV, R, LOGC, B, 0>(v, w[0], ps, false);
-        if (B + 1 >= LO && B + 1 < HI) rx_stage<INV, R, LOGC, B, 1>(v, w[1], ps, false);
-        if (B + 2 >= LO && B + 2 < HI) rx_stage<INV, R, LOGC, B, 2>(v, w[2], ps, false);
-        if (B + 3 >= LO && B + 3 < HI) rx_stage<INV, R, LOGC, B, 3>(v, w[3], ps, false);
+        if (B + 0 >= LO && B + 0 < HI) rx_stage<INV, R, LOGC, B, 0, SCALED>(v, w[0], ps, false);
+        if (B + 1 >= LO && B + 1 < HI) rx_stage<INV, R, LOGC, B, 1, SCALED>(v, w[1], ps, false);
+        if (B + 2 >= LO && B + 2 < HI) rx_stage<INV, R, LOGC, B, 2, SCALED>(v, w[2], ps, false);
+        if (B + 3 >= LO && B + 3 < HI) rx_stage<INV, R, LOGC, B, 3, SCALED>(v, w[3], ps, false);
     }
 }
 
@@ -307,8 +307,10 @@ __device__ __forceinline__ T* rx_sbase(T* p) {
 
 // FROM_REGS: the first group takes its 16 values from v instead of loading them (the fused
 // interpolate + extend kernel hands the coefficients over in registers).
-// SP (compile time): an inverse pass scales on store (ps.scale), a forward pass has a
+// SP (compile time): an inverse pass scales in its top stage (ps.scaled), a forward pass has a
 // zero-padded top stage (ps.dup_top): its values 8..15 are the zero partners, never read.
+// A strided forward pass stores its signed words as they are; the contiguous pass, always the
+// last one, stores canonical words.
 // Strided HBM accesses address the uniform column pointer plus a uniform row offset (rx_sbase)
 // with a 32-bit per-lane byte offset (words < 2^30), which the SGPR-base global forms take as is.
 template <bool INV, int R, int LOGC, int GI, bool SP, bool FROM_REGS = false>
@@ -363,7 +365,7 @@ __device__ __forceinline__ void rx_run(uint32_t (&v)[RX], const uint32_t (&w)[4]
             __syncthreads();
             rx_lds_get<LOGC, B>(v, lds, row0, lane);
         }
-        rx_group<INV, R, LOGC, B, S::LO, S::HI>(v, w, ps, DUP && GI == 0);
+        rx_group<INV, R, LOGC, B, S::LO, S::HI, INV && SP>(v, w, ps, DUP && GI == 0);
         if constexpr (GI + 1 < NG) {
             using SN = RxGroupShape<INV, R, GI + 1>;
             uint32_t wn[4][8];
@@ -373,9 +375,9 @@ __device__ __forceinline__ void rx_run(uint32_t (&v)[RX], const uint32_t (&w)[4]
             rx_run<INV, R, LOGC, GI + 1, SP, FROM_REGS>(v, wn, lds, src, dst, tower, ps, hi, r, lane, base);
         } else {
             const uint32_t g0 = base | (row0 << ps.s_lo) | lane;
-            if constexpr (INV && SP) {
+            if constexpr (!INV && LOGC == 0) {
 #pragma unroll
-                for (int k = 0; k < RX; k++) v[k] = mmul(v[k], ps.scale);
+                for (int k = 0; k < RX; k++) v[k] = mcanon(v[k]);
             }
             if constexpr (B == 0 && LOGC == 0) {
                 SR_GLOBAL u32x4* d4 = (SR_GLOBAL u32x4*)(dst + g0);
@@ -534,7 +536,7 @@ template <bool INV>
 static void rx_dispatch(uint32_t R, uint32_t logc, dim3 grid, dim3 block, size_t lds, hipStream_t st,
                         const uint32_t* const* src, uint32_t* const* dst, const uint32_t* tower, const RxPass& ps) {
     // the inverse's scaled pass and the forward's zero-padded top pass run the SP form
-    const bool sp = INV ? ps.scale != 1u : ps.dup_top != 0u;
+    const bool sp = INV ? ps.scaled != 0u : ps.dup_top != 0u;
 #define SR_RX(RR, CC)                                                                                       \
     if (R == RR && logc == CC) {                                                                            \
         if (sp)                                                                                             \
@@ -560,7 +562,7 @@ static void run_rx_pass(Ctx& c, bool inverse, const uint32_t* const* src, uint32
     SR_CHECK(blocks < (1ull << 31), "fft grid too large");
     SR_CHECK(R >= (uint32_t)RX_LOG && nt <= 512 && logc <= ps.s_lo && tile_log <= ps.m, "fft pass shape");
     SR_CHECK(logc != 0 || ps.s_lo == 0, "fft: contiguous pass must start at stage 0");
-    const uint32_t* tower = inverse ? c.d_itw2 : c.d_tw2;  // doubled: products via mmul_t2
+    const uint32_t* tower = inverse ? c.d_itw2 : c.d_tw2;  // signed doubled words (mtw2)
     KTimer kt(c,
               std::string(inverse ? "fft_ifft_pass" : "fft_lde_pass") + " m=" + std::to_string(ps.m) +
                   " R=" + std::to_string(R) + " C=" + std::to_string(1u << logc) + " cols=" + std::to_string(n_cols),
@@ -595,6 +597,16 @@ static std::vector<std::pair<uint32_t, uint32_t>> rx_plan(uint32_t m, uint32_t T
 }
 static uint32_t rx_logc(std::pair<uint32_t, uint32_t> p, uint32_t TILE_LOG) {
     return p.first == 0 ? 0u : std::min<uint32_t>(TILE_LOG - p.second, p.first);
+}
+
+// Last inverse pass: the scale 2^-m and its product with the top stage's twiddle, the inverse
+// x-coordinate of halfOdds(1) (the one entry of the tower's last layer, the same for every m).
+static void rx_set_scale(Ctx& c, RxPass& ps) {
+    const uint32_t n_inv = minv((uint32_t)((1ull << ps.m) % P));
+    const uint32_t t = minv(idx_to_point(c.gen, half_odds_initial(1)).x);
+    ps.scaled = 1;
+    ps.scale = mtw2(n_inv);
+    ps.scale_t = mtw2(mmul(n_inv, t));
 }
 
 static bool fused_dispatch(uint32_t R, uint32_t logc, dim3 grid, dim3 block, size_t lds, hipStream_t st,
@@ -636,7 +648,6 @@ void launch_circle_ifft_lde(Ctx& c, const uint32_t* const* d_eval, uint32_t* con
         return;
     }
     c.ensure_tower(m);
-    const uint32_t n_inv = minv((uint32_t)((1ull << n) % P));
     const size_t np = pi_plan.size();
     // inverse passes below the top one (evaluations -> d_coef, in place afterwards)
     for (size_t i = 0; i + 1 < np; i++) {
@@ -645,8 +656,6 @@ void launch_circle_ifft_lde(Ctx& c, const uint32_t* const* d_eval, uint32_t* con
         ps.src_log = n;
         ps.s_lo = pi_plan[i].first;
         ps.tower_log = c.tower_log;
-        ps.scale = 1u;
-        ps.dup_top = 0;
         run_rx_pass(c, true, i == 0 ? d_eval : (const uint32_t* const*)d_coef, d_coef, n_cols, pi_plan[i].second,
                     rx_logc(pi_plan[i], TILE_LOG), ps);
     }
@@ -658,12 +667,11 @@ void launch_circle_ifft_lde(Ctx& c, const uint32_t* const* d_eval, uint32_t* con
         pi.src_log = n;
         pi.s_lo = top.first;
         pi.tower_log = c.tower_log;
-        pi.scale = n_inv;
+        rx_set_scale(c, pi);
         pf.m = m;
         pf.src_log = m;
         pf.s_lo = top.first;
         pf.tower_log = c.tower_log;
-        pf.scale = 1u;
         const uint32_t tile_log = R + logc;
         SR_CHECK(R >= (uint32_t)RX_LOG && tile_log <= n && logc <= top.first, "fused fft pass shape");
         const uint32_t nt = 1u << (tile_log - RX_LOG);
@@ -689,8 +697,6 @@ void launch_circle_ifft_lde(Ctx& c, const uint32_t* const* d_eval, uint32_t* con
         ps.src_log = m;
         ps.s_lo = pp.first;
         ps.tower_log = c.tower_log;
-        ps.scale = 1u;
-        ps.dup_top = 0;
         run_rx_pass(c, false, (const uint32_t* const*)d_lde, d_lde, n_cols, pp.second, rx_logc(pp, TILE_LOG), ps);
     }
 }
@@ -730,12 +736,11 @@ void launch_circle_fft(Ctx& c, bool inverse, const uint32_t* const* d_src, uint3
     const std::vector<std::pair<uint32_t, uint32_t>> passes = rx_plan(m, TILE_LOG);  // (s_lo, R)
     auto logc_of = [&](std::pair<uint32_t, uint32_t> p) { return rx_logc(p, TILE_LOG); };
     auto mk = [&](std::pair<uint32_t, uint32_t> p, bool last) {
-        RxPass ps;
+        RxPass ps{};
         ps.m = m;
         ps.s_lo = p.first;
         ps.tower_log = c.tower_log;
-        ps.scale = (inverse && last) ? n_inv : 1u;
-        ps.dup_top = 0;
+        if (inverse && last) rx_set_scale(c, ps);
         return ps;
     };
     size_t np = passes.size();
@@ -771,7 +776,7 @@ __global__ void tower_kernel(uint32_t M, uint32_t* __restrict__ tw, uint32_t* __
     if (i == total - 1) {
         tw[i] = 1;
         itw[i] = 1;
-        tw2[i] = 2;
+        tw2[i] = 2;  // mtw2(1)
         itw2[i] = 2;
         return;
     }
@@ -787,8 +792,8 @@ __global__ void tower_kernel(uint32_t M, uint32_t* __restrict__ tw, uint32_t* __
     const uint32_t ix = minv(p.x);
     tw[i] = p.x;
     itw[i] = ix;
-    tw2[i] = p.x << 1;
-    itw2[i] = ix << 1;
+    tw2[i] = (uint32_t)mtw2(p.x);
+    itw2[i] = (uint32_t)mtw2(ix);
 }
 
 void launch_tower(Ctx& c, uint32_t log, uint32_t* d_tw, uint32_t* d_itw, uint32_t* d_tw2, uint32_t* d_itw2) {

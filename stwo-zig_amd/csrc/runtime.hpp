@@ -84,8 +84,8 @@ struct Ctx {
     uint64_t tower_builds = 0;  // builds of the tower since ctx_init
     uint32_t* d_tw = nullptr;
     uint32_t* d_itw = nullptr;
-    // The same towers doubled (2t as a plain u32 word, < 2^32): the register FFT multiplies by
-    // 2t so that b*t mod p reduces with one shift (mmul_t2).
+    // The same towers as signed doubled words (mtw2): the register FFT's products fold with
+    // one shift and need no reduction between stages (mbfly, mmul_s).
     uint32_t* d_tw2 = nullptr;
     uint32_t* d_itw2 = nullptr;
     // Completion counters of the tree-layer launches (zero between launches).

@@ -75,3 +75,35 @@ def test_m31_inverse(driver):
     assert [g[0] for g in got] == [pow(a, P - 2, P) for a in vals]
     assert all(g[0] * a % P == 1 for g, a in zip(got, vals))
     assert run(driver, ["i 0"]) == [(0,)]
+
+
+# words at the ends of the ranges the butterflies state, and twiddles around p / 2, where the
+# signed doubled word changes sign
+SIGNED = [-P, -P + 1, -(1 << 30) - 1, -(1 << 30), -2, -1, 0, 1, 2, (1 << 30) - 1, 1 << 30, P - 2, P - 1]
+TWIDDLES = [0, 1, 2, (P - 1) // 2 - 1, (P - 1) // 2, (P + 1) // 2, (P + 3) // 2, P - 2, P - 1]
+
+
+def test_signed_butterfly(driver):
+    """Forward butterfly: congruent to (a + b t, a - b t), and closed on [-p, p - 1]."""
+    rng = random.Random(31)
+    ops = [(a, b, t) for a in SIGNED for b in SIGNED for t in TWIDDLES]
+    ops += [(rng.randint(-P, P - 1), rng.randint(-P, P - 1), rng.randrange(P)) for _ in range(5000)]
+    for (a, b, t), (x, y, cx, cy) in zip(ops, run(driver, ["f %d %d %d" % v for v in ops])):
+        assert -P <= x <= P - 1 and -P <= y <= P - 1, (a, b, t)
+        assert (cx, cy) == ((a + b * t) % P, (a - b * t) % P), (a, b, t)
+        assert (x - cx) % P == 0 and (y - cy) % P == 0
+
+
+def test_inverse_butterflies_and_signed_product(driver):
+    """Inverse butterfly on words in [0, p] (p stands for 0), plain (a + b in [0, p], the product
+    canonical) and scaled (both canonical); the product of a signed word in [-p, p]."""
+    rng = random.Random(32)
+    words = sorted({abs(v) for v in SIGNED})
+    ops = [(a, b, t, s) for a in words for b in words for t in TWIDDLES for s in (1, (P + 1) // 2, P - 1)]
+    ops += [tuple(rng.randrange(P) for _ in range(4)) for _ in range(5000)]
+    for (a, b, t, s), (x, y, xs, ys) in zip(ops, run(driver, ["g %d %d %d %d" % v for v in ops])):
+        assert x <= P and x % P == (a + b) % P and y == (a - b) * t % P, (a, b, t)
+        assert (xs, ys) == ((a + b) * s % P, (a - b) * t * s % P), (a, b, t, s)
+    prods = [(d, t) for d in SIGNED + [P] for t in TWIDDLES]
+    got = run(driver, ["m %d %d" % v for v in prods])
+    assert [g[0] for g in got] == [d * t % P for d, t in prods]
