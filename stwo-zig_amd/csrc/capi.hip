@@ -458,7 +458,7 @@ int stwo_rocm_pow_grind(stwo_rocm_ctx* ctx, const uint8_t digest[32], uint32_t p
         if (pow_bits == 0) return;
         uint8_t prefix[32];
         ch.pow_prefix(pow_bits, prefix);
-        uint64_t chunk = pow_bits <= 16 ? (1ull << 20) : (1ull << 24);
+        const uint64_t chunk = pow_launch_nonces(pow_bits);
         for (uint64_t base = 0;; base += chunk) {
             uint64_t r = launch_pow_grind(c, prefix, pow_bits, base, chunk);
             if (r != UINT64_MAX) {

@@ -421,10 +421,8 @@ static uint64_t grind_one(Ctx& c, const Channel& ch, uint32_t pow_bits) {
     if (pow_bits == 0) return 0;
     uint8_t prefix[32];
     ch.pow_prefix(pow_bits, prefix);
-    // chunks are searched in order and each returns its lowest nonce, so the size only sets
-    // how much is ground past the first solution: ~16x the expected work, 2^12..2^26
-    const uint32_t cl = std::min(26u, std::max(12u, pow_bits + 4));
-    const uint64_t chunk = 1ull << cl;
+    // launches search their nonces in order and each returns its lowest valid one
+    const uint64_t chunk = pow_launch_nonces(pow_bits);
     for (uint64_t base = 0;; base += chunk) {
         uint64_t r = launch_pow_grind(c, prefix, pow_bits, base, chunk);
         if (r != UINT64_MAX) return r;

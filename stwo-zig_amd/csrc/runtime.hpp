@@ -420,6 +420,8 @@ void launch_xor_example_columns(Ctx& c, uint32_t log_size, uint32_t log_step, ui
 void launch_constant_composition(Ctx& c, uint32_t log_eval, const uint32_t v[4], uint32_t* const* out_coords);
 // PoW: lowest nonce in [base, base+count) or UINT64_MAX.
 uint64_t launch_pow_grind(Ctx& c, const uint8_t prefix[32], uint32_t bits, uint64_t base, uint64_t count);
+// Nonces one launch_pow_grind call should cover at a difficulty.
+uint64_t pow_launch_nonces(uint32_t bits);
 // The same for `batch` independent prefixes (d_prefix: 8 words each) over one nonce range:
 // d_best[k] (initialised by the caller to UINT64_MAX) receives prefix k's lowest valid nonce.
 void launch_pow_grind_batch(Ctx& c, const uint32_t* d_prefix, uint32_t batch, uint32_t bits, uint64_t base,

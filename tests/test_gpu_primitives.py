@@ -261,6 +261,16 @@ def test_pow_grind_matches_oracle(ctx, bits):
     assert ctx.grind(digest, bits) == oracle.pow_grind(digest, bits)
 
 
+@pytest.mark.parametrize("bits", [13, 17, 18, 19, 21])
+def test_pow_grind_lowest_nonce_over_strides(ctx, bits):
+    """Difficulties around the sizes of the thread count (2^14 .. 2^19 threads, several nonces per
+    thread): the nonce is the lowest valid one, for digests whose solutions fall in different strides."""
+    for k in range(4):
+        digest = hashlib.blake2s(b"stride%d-%d" % (bits, k)).digest()
+        _say("pow", bits, k)
+        assert ctx.grind(digest, bits) == oracle.pow_grind(digest, bits)
+
+
 @pytest.mark.parametrize("log_n,seq,mode", [(5, 16, 0), (12, 100, 1), (20, 100, 0)])
 def test_widefib_trace_matches_oracle(ctx, log_n, seq, mode):
     d = ctx.alloc(4 * seq << log_n)
