@@ -15,6 +15,8 @@
 // levels of any tree from hashes already in HBM.
 // fri_tail: the layers below FRI_TAIL_MAX_LOG + 1 in one workgroup with the line and the
 // hash level resident in LDS.
+#include <type_traits>
+
 #include "chan.hpp"
 
 namespace sr {
@@ -83,13 +85,25 @@ __global__ __launch_bounds__(256) void fold_circle_kernel(const uint32_t* __rest
 
 // ---------------------------------------------------------------------------
 // Tree levels inside one workgroup.  A level of c <= 128 parents uses one quad of lanes per
-// compression (blake2s_quad.hpp: about half the latency of a one-lane compression while a
-// SIMD runs one wave); wider levels use one lane per compression, which does the same
-// work in fewer instructions once the SIMDs are full.  Shared by the layer and tail kernels.
+// compression (blake2s_quad.hpp); wider levels use one lane per compression, which does the
+// same work in fewer instructions once the SIMDs are full.  A quad level's hashes go to the
+// next level through a board in LDS (words in lane order).  From 16 parents on the quads of
+// wave 0 are enough, and LDS serves its accesses in order: no barrier until the root.
+// Shared by the layer and tail kernels.
 
 constexpr uint32_t TL_THREADS = 256;    // tree-layer workgroup: one wave per SIMD
-constexpr uint32_t TAIL_THREADS = 1024;  // tail workgroup: a whole line of 2^10 values
+constexpr uint32_t TAIL_THREADS = 512;   // tail workgroup: two waves per SIMD keep it issuing on the wide layers
 constexpr uint32_t TR_QUAD_MAX = 128;    // widest level hashed by quads
+constexpr uint32_t TR_WAVE_MAX = 16;     // widest level hashed by the quads of one wave
+constexpr uint32_t TR_BOARD = 64;        // messages of the widest level that reads the board
+
+// LDS of the levels: plain hashes (8 words each) of the one-lane levels, hA then hB, or the
+// board of the quad levels over the same words (a level's inputs are all read before its board
+// is written); the channel's boards lie before them.
+constexpr uint32_t TR_PLAIN_A = 1024 * 8, TR_PLAIN_B = 512 * 8;
+constexpr uint32_t TR_LEVEL_WORDS = TR_PLAIN_A + TR_PLAIN_B;
+static_assert(TR_LEVEL_WORDS >= 160 * TR_BOARD, "plain hashes and the board share their words");
+constexpr uint32_t TR_CHAN_WORDS = 2 * 160;
 
 __device__ __forceinline__ void tr_load16(const uint32_t* in, uint32_t m[16]) {
     const uint4* m4 = (const uint4*)in;
@@ -100,10 +114,7 @@ __device__ __forceinline__ void tr_load16(const uint32_t* in, uint32_t m[16]) {
     }
 }
 
-__device__ __forceinline__ void tr_put_quad(uint32_t* lds, uint8_t* __restrict__ g, uint32_t q, uint32_t hlo,
-                                            uint32_t hhi) {
-    lds[q] = hlo;
-    lds[4 + q] = hhi;
+__device__ __forceinline__ void tr_store_quad(uint8_t* __restrict__ g, uint32_t q, uint32_t hlo, uint32_t hhi) {
     uint32_t* o = (uint32_t*)g;
     o[q] = hlo;
     o[4 + q] = hhi;
@@ -118,40 +129,107 @@ __device__ __forceinline__ void tr_put_lane(uint32_t* lds, uint8_t* __restrict__
     o[1] = y;
 }
 
-// Parents p < c of the 2c child hashes in `in` (LDS, 8 words per hash), written to `out`
-// (LDS) and to the tree level `gl` at hashes first + p (layers.zig:99-140:
-// H(node_seed; left || right)).  The level of one parent (c == 1) runs on quad 0, which is
-// left holding it as (rlo, rhi) = words (q, 4 + q).  Ends with a workgroup barrier.
+// Per-lane constants of the quad levels.
+struct TrQuad {
+    uint32_t t, q;
+    QuadLane L;
+    QuadIo io;
+    uint32_t nlo, nhi;  // node seed words q, 4 + q
+    __device__ __forceinline__ TrQuad(uint32_t t_, const B2State& node_seed)
+        : t(t_), q(t_ & 3), L(t_ & 3), io(t_ >> 2, t_ & 3) {
+        nlo = L.sel(node_seed.h[0], node_seed.h[1], node_seed.h[2], node_seed.h[3]);
+        nhi = L.sel(node_seed.h[4], node_seed.h[5], node_seed.h[6], node_seed.h[7]);
+    }
+};
+
+// Address of hash `first` of tree level `lev`.
+__device__ __forceinline__ uint8_t* tr_at(uint8_t* tree, uint32_t lev, uint64_t first) {
+    return tree + ((((uint64_t)1 << lev) - 1) + first) * 32;
+}
+
+// The levels of c, c/2, ..., 1 parents by quads; the 2c children are on the board, written by
+// quads 0 .. 2c - 1.  Level `lev` has c parents of this workgroup, from parent blk * c on.  The
+// root ends as (rlo, rhi) = words (q, 4 + q) in quads 0 and 1 (the channel step takes it from
+// both).  Waves other than the first leave once the first is alone with the rest.
+__device__ __forceinline__ void tr_quad_levels(const TrQuad& Q, uint32_t* board, uint32_t c, uint8_t* tree,
+                                               uint32_t lev, uint64_t blk, uint32_t& rlo, uint32_t& rhi) {
+    const uint32_t p = Q.t >> 2;
+    for (;; c >>= 1, lev--) {
+        if (2 * c > TR_WAVE_MAX) __syncthreads();
+        else if (Q.t >= 64) return;
+        else qboard_wave_fence();
+        if (p < c || (c == 1 && p == 1)) {
+            rlo = Q.nlo;
+            rhi = Q.nhi;
+            qboard_compress<TR_BOARD>(Q.L, rlo, rhi, board, c == 1 ? 16 * Q.q : Q.io.rd, 128, true);
+        }
+        if (c > TR_WAVE_MAX) __syncthreads();  // every message is read
+        if (p < c) {
+            if (c > 1) qboard_put<TR_BOARD>(board, Q.io, rlo, rhi);
+            tr_store_quad(tr_at(tree, lev, blk * c) + 32 * p, Q.q, rlo, rhi);
+        }
+        if (c == 1) return;
+    }
+}
+
+// From 2c hashes, plain in hA (their writes are behind a barrier) or, if `on_board`, on the board:
+// the one-lane levels between hA and hB, a first quad level that selects its message words, then
+// the levels on the board, which may overlap that level's inputs.
 template <uint32_t T>
-__device__ __forceinline__ void tr_level(const uint32_t* in, uint32_t* out, uint32_t c, uint8_t* __restrict__ gl,
-                                         uint64_t first, const B2State& seed, uint32_t t, uint32_t& rlo,
-                                         uint32_t& rhi) {
-    if (c <= TR_QUAD_MAX) {
-        const uint32_t q = t & 3;
-        const QuadLane L(q);
-        for (uint32_t p = t >> 2; p < c; p += T / 4) {
-            uint32_t m[16];
-            tr_load16(in + 16 * p, m);
-            uint32_t hlo = L.sel(seed.h[0], seed.h[1], seed.h[2], seed.h[3]);
-            uint32_t hhi = L.sel(seed.h[4], seed.h[5], seed.h[6], seed.h[7]);
-            b2_compress_quad(L, hlo, hhi, m, 128, true);
-            tr_put_quad(out + 8 * p, gl + (first + p) * 32, q, hlo, hhi);
-            if (p == 0) {
-                rlo = hlo;
-                rhi = hhi;
+__device__ __forceinline__ void tr_levels(const TrQuad& Q, uint32_t* lds, bool on_board, uint32_t c, uint8_t* tree,
+                                          uint32_t lev, uint64_t blk, const B2State& seed, uint32_t& rlo,
+                                          uint32_t& rhi) {
+    if (!on_board) {
+        uint32_t *in = lds, *out = lds + TR_PLAIN_A;
+        for (; c > TR_QUAD_MAX; c >>= 1, lev--) {
+            uint8_t* g = tr_at(tree, lev, blk * c);
+            for (uint32_t p = Q.t; p < c; p += T) {
+                uint32_t m[16], h[8];
+                tr_load16(in + 16 * p, m);
+#pragma unroll
+                for (int k = 0; k < 8; k++) h[k] = seed.h[k];
+                b2_compress(h, m, 128, true);
+                tr_put_lane(out + 8 * p, g + 32 * p, h);
+            }
+            __syncthreads();
+            uint32_t* x = in;
+            in = out;
+            out = x;
+        }
+        constexpr uint32_t STEP = T / 4, IT = (TR_QUAD_MAX + STEP - 1) / STEP;
+        uint32_t lo[IT], hi[IT];
+#pragma unroll
+        for (uint32_t k = 0; k < IT; k++) {
+            lo[k] = Q.nlo;
+            hi[k] = Q.nhi;
+        }
+        // one copy of the compression's code
+#pragma unroll 1
+        for (uint32_t k = 0; k < IT; k++) {
+            const uint32_t p = (Q.t >> 2) + k * STEP;
+            if (p < c || (c == 1 && p == 1)) {
+                uint32_t m[16], hlo = Q.nlo, hhi = Q.nhi;
+                tr_load16(in + (c == 1 ? 0 : 16 * p), m);
+                b2_compress_quad(Q.L, hlo, hhi, m, 128, true);
+                if (p < c) tr_store_quad(tr_at(tree, lev, blk * c) + 32 * p, Q.q, hlo, hhi);
+#pragma unroll
+                for (uint32_t i = 0; i < IT; i++) {
+                    lo[i] = i == k ? hlo : lo[i];
+                    hi[i] = i == k ? hhi : hi[i];
+                }
             }
         }
-    } else {
-        for (uint32_t p = t; p < c; p += T) {
-            uint32_t m[16], h[8];
-            tr_load16(in + 16 * p, m);
+        rlo = lo[0];
+        rhi = hi[0];
+        if (c == 1) return;
+        __syncthreads();
 #pragma unroll
-            for (int k = 0; k < 8; k++) h[k] = seed.h[k];
-            b2_compress(h, m, 128, true);
-            tr_put_lane(out + 8 * p, gl + (first + p) * 32, h);
-        }
+        for (uint32_t k = 0; k < IT; k++)
+            if ((Q.t >> 2) + k * STEP < c) qboard_put<TR_BOARD>(lds, Q.io, lo[k], hi[k], k * STEP / 2);
+        c >>= 1;
+        lev--;
     }
-    __syncthreads();
+    tr_quad_levels(Q, lds, c, tree, lev, blk, rlo, rhi);
 }
 
 // Leaf hash of one QM31 value (leaf_qm31 above) by a quad, the value in every lane.
@@ -188,30 +266,67 @@ __device__ __forceinline__ qm31 tr_fold_at(const FriLayerArgs& a, uint64_t i, qm
     }
 }
 
-// Channel step on a root held by quad 0 as (rlo, rhi), the channel digest `dg` in registers
-// of every lane of the quad (MerkleChannel.mixRoot then drawSecureFelt, as
-// chan_mix_root_draw_quad): updates dg and the DevChannel, copies the root to root_out.
-__device__ __forceinline__ qm31 tr_chan_step(const QuadLane& L, uint32_t q, uint32_t dg[8], uint32_t rlo, uint32_t rhi,
+// The channel in LDS: two one-slot boards, the message of mixRoot (digest || root) and that of
+// drawSecureFelt (digest || draw counter || zeros).  All threads; the caller's barrier ends it.
+template <uint32_t T>
+__device__ __forceinline__ void tr_chan_init(const TrQuad& Q, uint32_t* chan, const DevChannel* ch) {
+    if (Q.t >= 64) {
+        for (uint32_t i = Q.t - 64; i < 160; i += T - 64) chan[160 + i] = 0;
+    } else if (Q.t < 4) {
+        qboard_put<1>(chan, Q.io, ch->digest[Q.q], ch->digest[4 + Q.q]);
+    }
+}
+
+// Channel step on a root held by quads 0 and 1 (the threads that run it) as (rlo, rhi)
+// (MerkleChannel.mixRoot then drawSecureFelt, as chan_mix_root_draw_quad): updates the LDS
+// messages and the DevChannel, copies the root to root_out.
+__device__ __forceinline__ qm31 tr_chan_step(const TrQuad& Q, uint32_t* chan, uint32_t rlo, uint32_t rhi,
                                              DevChannel* __restrict__ ch, uint32_t* __restrict__ root_out) {
-    uint32_t pay[16] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    quad_gather8(rlo, rhi, pay);
-    if (root_out) {
-        root_out[q] = rlo;
-        root_out[4 + q] = rhi;
+    const QuadLane& L = Q.L;
+    const uint32_t ilo = L.sel(SR_B2_IV0 ^ 0x01010020u, SR_B2_IV1, SR_B2_IV2, SR_B2_IV3);
+    const uint32_t ihi = L.sel(SR_B2_IV4, SR_B2_IV5, SR_B2_IV6, SR_B2_IV7);
+    uint32_t *const mix = chan, *const draw = chan + 160;
+    if (Q.t >= 4) qboard_put<1>(mix, Q.io, rlo, rhi);
+    uint32_t dlo = 0, dhi = 0;
+    // compression 0 is the mix, the others are draws (more than one with probability ~2^-28)
+#pragma unroll 1
+    for (uint32_t k = 0; k <= 64; k++) {
+        qboard_wave_fence();
+        uint32_t hlo = ilo, hhi = ihi;
+        qboard_compress<1>(L, hlo, hhi, k ? draw : mix, 16 * Q.q, k ? 37 : 64, true);
+        if (k == 0) {
+            dlo = hlo;
+            dhi = hhi;
+            if (Q.t < 4) qboard_put<1>(draw, Q.io, dlo, dhi);
+            continue;
+        }
+        uint32_t bad = (hlo >= 2u * P || hhi >= 2u * P) ? 1u : 0u;
+        bad |= quad_perm<QP_ROT1>(bad);
+        bad |= quad_perm<QP_ROT2>(bad);  // OR over the quad (the same in both)
+        // message word 8, the draw counter (the first word of the second half): the next one, or
+        // zero again for the next step
+        if ((bad || k > 1) && Q.t == 4) {
+#pragma unroll
+            for (int r = 0; r < 10; r++) *(uint32_t*)((uint8_t*)draw + 64 * r + Q.io.wr[2 * r]) = bad ? k : 0u;
+        }
+        if (bad) continue;
+        const qm31 a = {{mred64(quad_bcast<0>(hlo)), mred64(quad_bcast<1>(hlo))},
+                        {mred64(quad_bcast<2>(hlo)), mred64(quad_bcast<3>(hlo))}};
+        if (Q.t < 4) {
+            qboard_put<1>(mix, Q.io, dlo, dhi);
+            if (root_out) tr_store_quad((uint8_t*)root_out, Q.q, rlo, rhi);
+            ch->digest[Q.q] = dlo;
+            ch->digest[4 + Q.q] = dhi;
+            if (Q.q == 0) {
+                ch->n_draws = k;
+                qstore(a, ch->alpha);
+                qstore(qsqr(a), ch->alpha2);
+            }
+        }
+        return a;
     }
-    qchan_mix(L, dg, pay, 8);
-    uint32_t nd = 0, st = 0;
-    const qm31 a = qchan_draw(L, dg, nd, st);
-    // lane q stores digest words q and 4 + q (the digest is in every lane)
-    ch->digest[q] = L.sel(dg[0], dg[1], dg[2], dg[3]);
-    ch->digest[4 + q] = L.sel(dg[4], dg[5], dg[6], dg[7]);
-    if (q == 0) {
-        ch->n_draws = nd;
-        qstore(a, ch->alpha);
-        qstore(qsqr(a), ch->alpha2);
-        if (st) ch->status = 1;
-    }
-    return a;
+    if (Q.t == 0) ch->status = 1;
+    return qzero();
 }
 
 // One tree (or its top levels) in one launch.  Workgroup b owns the 2^s hashes
@@ -239,30 +354,38 @@ __global__ __launch_bounds__(TL_THREADS) void tree_layer_kernel(FriLayerArgs a0)
         a.cnt += (uint64_t)blockIdx.y * TREE_CNT_WORDS;
         a.xr += (uint64_t)blockIdx.y * TREE_CNT_WORDS;
     }
-    __shared__ __align__(16) uint32_t hA[1024 * 8];
-    __shared__ __align__(16) uint32_t hB[512 * 8];
+    __shared__ __align__(16) uint32_t sh[TR_CHAN_WORDS + TR_LEVEL_WORDS];
     __shared__ uint32_t last;
+    uint32_t *const chan = sh, *const lds = sh + TR_CHAN_WORDS;
     const uint32_t t = threadIdx.x, q = t & 3;
-    const QuadLane L(q);
+    const TrQuad Q(t, a.node_seed);
     const uint32_t n1 = 1u << a.s;
     const uint64_t base = (uint64_t)blockIdx.x * n1;
     uint8_t* lev_k0 = a.tree + (((uint64_t)1 << a.k0) - 1) * 32;
+    uint32_t rlo = 0, rhi = 0;
+    bool boards = false;  // the hashes of level k0 are on the board
     if constexpr (SRC == FRI_SRC_HASHES) {
         for (uint32_t p = t; p < n1; p += TL_THREADS) {
             const uint4* s4 = (const uint4*)(lev_k0 + (base + p) * 32);
             const uint4 x = s4[0], y = s4[1];
-            *(uint4*)&hA[8 * p] = x;
-            *(uint4*)&hA[8 * p + 4] = y;
+            *(uint4*)&lds[8 * p] = x;
+            *(uint4*)&lds[8 * p + 4] = y;
         }
     } else {
         const qm31 alpha = qload(a.ch->alpha);
-        if (n1 <= TR_QUAD_MAX) {
-            for (uint32_t p = t >> 2; p < n1; p += TL_THREADS / 4) {
-                const qm31 r = tr_fold_at<SRC>(a, base + p, alpha);
-                if (q == 0) a.dst_line[base + p] = make_uint4(r.c0.a, r.c0.b, r.c1.a, r.c1.b);
-                uint32_t hlo, hhi;
-                tr_leaf_quad(L, a.leaf_seed, r, hlo, hhi);
-                tr_put_quad(hA + 8 * p, lev_k0 + (base + p) * 32, q, hlo, hhi);
+        boards = n1 <= TR_QUAD_MAX;
+        if (boards) {
+#pragma unroll
+            for (uint32_t k = 0; k < TR_QUAD_MAX / (TL_THREADS / 4); k++) {
+                const uint32_t p = (t >> 2) + k * (TL_THREADS / 4);
+                if (p < n1) {
+                    const qm31 r = tr_fold_at<SRC>(a, base + p, alpha);
+                    if (q == 0) a.dst_line[base + p] = make_uint4(r.c0.a, r.c0.b, r.c1.a, r.c1.b);
+                    uint32_t hlo, hhi;
+                    tr_leaf_quad(Q.L, a.leaf_seed, r, hlo, hhi);
+                    qboard_put<TR_BOARD>(lds, Q.io, hlo, hhi, k * (TL_THREADS / 8));
+                    tr_store_quad(lev_k0 + (base + p) * 32, q, hlo, hhi);
+                }
             }
         } else {
             for (uint32_t p = t; p < n1; p += TL_THREADS) {
@@ -270,32 +393,29 @@ __global__ __launch_bounds__(TL_THREADS) void tree_layer_kernel(FriLayerArgs a0)
                 a.dst_line[base + p] = make_uint4(r.c0.a, r.c0.b, r.c1.a, r.c1.b);
                 uint32_t h[8];
                 tr_leaf_lane(a.leaf_seed, r, h);
-                tr_put_lane(hA + 8 * p, lev_k0 + (base + p) * 32, h);
+                tr_put_lane(lds + 8 * p, lev_k0 + (base + p) * 32, h);
             }
         }
     }
-    __syncthreads();
-    uint32_t rlo = 0, rhi = 0;
-    uint32_t *in = hA, *out = hB;
-    uint32_t lev = a.k0;
-    for (uint32_t c = n1 >> 1; c >= 1; c >>= 1) {
-        lev--;
-        tr_level<TL_THREADS>(in, out, c, a.tree + (((uint64_t)1 << lev) - 1) * 32, (uint64_t)blockIdx.x * c,
-                             a.node_seed, t, rlo, rhi);
-        uint32_t* x = in;
-        in = out;
-        out = x;
-    }
     const uint32_t nb = gridDim.x;
-    uint32_t dg[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (nb > 1) {
-        // Hand-off without an L2 writeback: lanes 0..7 publish the subtree root (in LDS since
-        // the barrier that ended the last level) with device-coherent stores (agent-scope
-        // atomic stores, global_store sc1), the wave waits until they are acknowledged, and
-        // thread 0 counts the workgroup; the last workgroup reads the roots with
-        // device-coherent loads.  The tree's own copy of the roots (plain stores) is read by
-        // later launches only.
-        if (t < 8) __hip_atomic_store(&a.xr[8 * blockIdx.x + t], in[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // nothing of the top pass is kept for the first one: the channel's boards are written by the
+    // workgroup that reaches the root
+    uint32_t c = n1 >> 1, lev = a.k0 - 1;
+    uint64_t blk = blockIdx.x;
+    for (bool top = nb == 1;; top = true) {
+        if (top && a.ch) tr_chan_init<TL_THREADS>(Q, chan, a.ch);
+        if (!boards || top) __syncthreads();
+        tr_levels<TL_THREADS>(Q, lds, boards, c, a.tree, lev, blk, a.node_seed, rlo, rhi);
+        if (top) break;
+        // Hand-off without an L2 writeback: quad 0 publishes the subtree root with
+        // device-coherent stores (agent-scope atomic stores, global_store sc1), the wave waits
+        // until they are acknowledged, and thread 0 counts the workgroup; the last workgroup
+        // reads the roots with device-coherent loads.  The tree's own copy of the roots (plain
+        // stores) is read by later launches only.
+        if (t < 4) {
+            __hip_atomic_store(&a.xr[8 * blockIdx.x + q], rlo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&a.xr[8 * blockIdx.x + 4 + q], rhi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         if (t < 64) {
             __builtin_amdgcn_s_waitcnt(0);
             if (t == 0) {
@@ -314,44 +434,28 @@ __global__ __launch_bounds__(TL_THREADS) void tree_layer_kernel(FriLayerArgs a0)
         // before its count).  One fence per launch, in the last workgroup only.
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         if (t <= TREE_CNT_GROUPS) atomicExch(&a.cnt[TREE_CNT_STRIDE * t], 0u);
-        if (a.ch && t < 4) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) dg[k] = a.ch->digest[k];
-        }
         // top levels from the nb subtree roots
         for (uint32_t i = t; i < 8 * nb; i += TL_THREADS)
-            hA[i] = __hip_atomic_load(&a.xr[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        in = hA;
-        out = hB;
-        for (uint32_t c = nb >> 1; c >= 1; c >>= 1) {
-            lev--;
-            tr_level<TL_THREADS>(in, out, c, a.tree + (((uint64_t)1 << lev) - 1) * 32, 0, a.node_seed, t, rlo, rhi);
-            uint32_t* x = in;
-            in = out;
-            out = x;
-        }
-    } else if (a.ch && t < 4) {
-#pragma unroll
-        for (int k = 0; k < 8; k++) dg[k] = a.ch->digest[k];
+            lds[i] = __hip_atomic_load(&a.xr[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        boards = false;
+        c = nb >> 1;
+        lev = a.k0 - a.s - 1;
+        blk = 0;
     }
-    // quad 0 holds the root
-    if (t < 4) {
-        if (a.ch) {
-            (void)tr_chan_step(L, q, dg, rlo, rhi, a.ch, a.root_out);
-        } else if (a.root_out) {
-            a.root_out[q] = rlo;
-            a.root_out[4 + q] = rhi;
-        }
+    if (a.ch) {
+        if (t < 8) (void)tr_chan_step(Q, chan, rlo, rhi, a.ch, a.root_out);
+    } else if (t < 4 && a.root_out) {
+        tr_store_quad((uint8_t*)a.root_out, q, rlo, rhi);
     }
 }
 
 // fri_tail: the inner layers below the committed line top_log (<= FRI_TAIL_MAX_LOG + 1) run
 // in one workgroup with the current line and hash level resident in LDS and the channel
-// digest in registers of quad 0: per layer the fold into the next line, its leaf hashes,
+// messages on LDS boards: per layer the fold into the next line, its leaf hashes,
 // the parent levels (layers.zig:99-140) and the channel step on the root, separated by
 // workgroup barriers instead of kernel boundaries (prover/fri.zig:377-621 runs the same
-// sequence per layer).  The last fold (into last_log) stores the line only.
+// sequence per layer).  The last fold (into last_log) stores the line only.  Layers of at most
+// 16 values run in the first wave alone, without a barrier.
 __global__ __launch_bounds__(TAIL_THREADS) void fri_tail_kernel(const FriTailArgs a) {
     // The per-log pointer arrays are read from the kernel arguments with the (uniform) log as
     // index and proof blockIdx.x's offset added at each use: a local copy of the arguments
@@ -361,70 +465,93 @@ __global__ __launch_bounds__(TAIL_THREADS) void fri_tail_kernel(const FriTailArg
     const auto at = [boff](auto* p) { return (decltype(p))((uint8_t*)p + boff); };
     DevChannel* __restrict__ ch = at(a.ch);
     const B2State leaf_seed = a.leaf_seed, node_seed = a.node_seed;
-    __shared__ __align__(16) uint32_t hA[TAIL_THREADS * 8];
-    __shared__ __align__(16) uint32_t hB[TAIL_THREADS / 2 * 8];
-    __shared__ uint4 vs[TAIL_THREADS];  // current line
-    __shared__ uint32_t sa[4];          // alpha
+    constexpr uint32_t NV = 1u << FRI_TAIL_MAX_LOG, PER = NV / TAIL_THREADS;
+    static_assert(TAIL_THREADS / 4 >= TR_QUAD_MAX, "a quad per value of a narrow layer");
+    __shared__ __align__(16) uint32_t sh[TR_CHAN_WORDS + TR_LEVEL_WORDS + 4 * NV + 4];
+    uint32_t *const chan = sh, *const lds = sh + TR_CHAN_WORDS;
+    uint4* const vs = (uint4*)(lds + TR_LEVEL_WORDS);  // current line
+    uint32_t* const sa = (uint32_t*)(vs + NV);         // alpha
     const uint32_t t = threadIdx.x, q = t & 3;
-    const QuadLane L(q);
+    const TrQuad Q(t, node_seed);
     uint32_t l = a.top_log;
     qm31 alpha = qload(ch->alpha);
-    uint32_t dg[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (t < 4) {
+    tr_chan_init<TAIL_THREADS>(Q, chan, ch);
+    // This thread's value k of a layer of n values: its quad's on narrow layers, else its lane's.
+    // The inverse x of the next layer's are loaded while this one's tree is hashed.
+    uint32_t inv[PER];
+    const auto value = [&](uint32_t n, uint32_t k) {
+        return n <= TR_QUAD_MAX ? (k ? n : t >> 2) : t + k * TAIL_THREADS;
+    };
+    const auto load_inv = [&](uint32_t log) {
+        const uint32_t n = 1u << (log - 1);
+        const uint32_t* inv_x = a.itw_half - ((size_t)1 << log);
 #pragma unroll
-        for (int k = 0; k < 8; k++) dg[k] = ch->digest[k];
-    }
+        for (uint32_t k = 0; k < PER; k++) inv[k] = value(n, k) < n ? inv_x[value(n, k)] : 0u;
+    };
+    load_inv(l);
+    __syncthreads();
     bool first = true;
     for (;;) {
         const uint32_t n = 1u << (l - 1);
-        const uint32_t* inv_x = a.itw_half - ((size_t)1 << l);
-        qm31 r = qzero();
-        if (t < n) {
-            const uint4* __restrict__ src = at(a.lines[l]);
-            const uint4 x = first ? src[2 * t] : vs[2 * t];
-            const uint4 y = first ? src[2 * t + 1] : vs[2 * t + 1];
-            r = tr_fold(x, y, alpha, inv_x[t]);
+        const bool quads = n <= TR_QUAD_MAX;
+        qm31 r[PER];
+#pragma unroll
+        for (uint32_t k = 0; k < PER; k++) {
+            const uint32_t p = value(n, k);
+            if (p < n) {
+                const uint4* __restrict__ src = at(a.lines[l]);
+                const uint4 x = first ? src[2 * p] : vs[2 * p];
+                const uint4 y = first ? src[2 * p + 1] : vs[2 * p + 1];
+                r[k] = tr_fold(x, y, alpha, inv[k]);
+            }
         }
         first = false;
-        __syncthreads();
+        if (n <= TR_WAVE_MAX) qboard_wave_fence();
+        else __syncthreads();
         l--;
-        const uint4 rv = make_uint4(r.c0.a, r.c0.b, r.c1.a, r.c1.b);
-        if (t < n) {
-            vs[t] = rv;
-            at(a.lines[l])[t] = rv;
+#pragma unroll
+        for (uint32_t k = 0; k < PER; k++) {
+            const uint32_t p = value(n, k);
+            if (p < n && (!quads || q == 0)) {
+                const uint4 rv = make_uint4(r[k].c0.a, r[k].c0.b, r[k].c1.a, r[k].c1.b);
+                vs[p] = rv;
+                at(a.lines[l])[p] = rv;
+            }
         }
         if (l == a.last_log) break;
+        load_inv(l);
         uint8_t* tree = at(a.trees[l]);
         uint8_t* leaves = tree + (((size_t)1 << l) - 1) * 32;
-        if (n <= TR_QUAD_MAX) {
-            __syncthreads();
-            for (uint32_t p = t >> 2; p < n; p += TAIL_THREADS / 4) {
-                const uint4 v = vs[p];
-                uint32_t hlo, hhi;
-                tr_leaf_quad(L, leaf_seed, qm31{{v.x, v.y}, {v.z, v.w}}, hlo, hhi);
-                tr_put_quad(hA + 8 * p, leaves + (size_t)p * 32, q, hlo, hhi);
-            }
-        } else if (t < n) {
-            uint32_t h[8];
-            tr_leaf_lane(leaf_seed, r, h);
-            tr_put_lane(hA + 8 * t, leaves + (size_t)t * 32, h);
-        }
-        __syncthreads();
         uint32_t rlo = 0, rhi = 0;
-        uint32_t *in = hA, *out = hB;
-        uint32_t lev = l;
-        for (uint32_t c = n >> 1; c >= 1; c >>= 1) {
-            lev--;
-            tr_level<TAIL_THREADS>(in, out, c, tree + (((size_t)1 << lev) - 1) * 32, 0, node_seed, t, rlo, rhi);
-            uint32_t* x = in;
-            in = out;
-            out = x;
+        if (quads) {
+            const uint32_t p = t >> 2;
+            if (p < n) {
+                uint32_t hlo, hhi;
+                tr_leaf_quad(Q.L, leaf_seed, r[0], hlo, hhi);
+                qboard_put<TR_BOARD>(lds, Q.io, hlo, hhi);
+                tr_store_quad(leaves + (size_t)p * 32, q, hlo, hhi);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < PER; k++) {
+                const uint32_t p = value(n, k);
+                if (p < n) {
+                    uint32_t h[8];
+                    tr_leaf_lane(leaf_seed, r[k], h);
+                    tr_put_lane(lds + 8 * p, leaves + (size_t)p * 32, h);
+                }
+            }
+            __syncthreads();
         }
-        if (t < 4) {
-            const qm31 na = tr_chan_step(L, q, dg, rlo, rhi, ch, a.roots[l] ? at(a.roots[l]) : nullptr);
-            if (t == 0) qstore(na, sa);
+        tr_levels<TAIL_THREADS>(Q, lds, quads, n >> 1, tree, l - 1, 0, node_seed, rlo, rhi);
+        if (t < 8) {
+            alpha = tr_chan_step(Q, chan, rlo, rhi, ch, a.roots[l] ? at(a.roots[l]) : nullptr);
+            if (t == 0) qstore(alpha, sa);
         }
-        __syncthreads();
+        // the next layer folds in the first wave only if it has at most 16 values
+        if (n > 2 * TR_WAVE_MAX) __syncthreads();
+        else if (t >= 64) return;
+        else qboard_wave_fence();
         alpha = qload(sa);
     }
 }

@@ -187,6 +187,13 @@ def test_commit_fri_layers(ctx, log_size, last_log):
         x.close() if hasattr(x, "close") else x.free()
 
 
+@pytest.mark.parametrize("log_size,last_log", [(3, 1), (4, 1), (5, 3), (6, 1), (7, 5), (8, 1), (9, 7), (10, 1),
+                                               (11, 9), (16, 1)])
+def test_commit_fri_layers_at_tail_edges(ctx, log_size, last_log):
+    """The one-workgroup tail entered at every width (one wave, quads, one-lane hashes) and left early."""
+    test_commit_fri_layers(ctx, log_size, last_log)
+
+
 def test_gather_values_lifted(ctx):
     rng = np.random.default_rng(5)
     logs = [3, 6, 6, 9]

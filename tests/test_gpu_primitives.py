@@ -144,6 +144,24 @@ def test_merkle_every_level_matches_oracle(ctx, log):
         b.free()
 
 
+@pytest.mark.parametrize("log", [1, 2, 3, 4, 5, 6, 7, 8, 10, 11, 12, 16, 17])
+def test_merkle_whole_tree_at_every_split(ctx, log):
+    """Every hash of the tree where the top reduction changes form: one parent, levels of one wave,
+    of several waves, of one-lane hashes; one and several workgroups."""
+    rng = np.random.default_rng(100 + log)
+    cols = rand_cols(rng, 2, log)
+    bufs = [ctx.to_device(c) for c in cols]
+    _say("merkle whole tree", log)
+    tree = ctx.commit_merkle([b.ptr for b in bufs], [log] * 2)
+    root, layers = oracle.merkle_commit(cols)
+    assert tree.root == root
+    for lay in range(log + 1):
+        assert b"".join(tree.read_hashes(lay, list(range(1 << lay)))) == bytes(layers[lay]), lay
+    tree.free()
+    for b in bufs:
+        b.free()
+
+
 @pytest.mark.parametrize("n_cols,log", [(0, 0), (1, 1), (1, 2), (3, 3), (5, 6), (16, 8), (17, 8), (2, 10), (2, 11),
                                         (100, 14), (8, 21)])
 def test_merkle_uniform_matches_oracle(ctx, n_cols, log):
