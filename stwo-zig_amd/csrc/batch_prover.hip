@@ -102,7 +102,7 @@ BatchPlan* batch_plan_create(Ctx& c, const ProveParams& prm, uint32_t K) {
     const uint32_t L = n + B;
     const uint32_t last_log = prm.log_last_layer_degree_bound + B;
     SR_CHECK(L > last_log, "trace too small for the FRI configuration");
-    SR_CHECK(L - 1 <= TREE_LAYER_MAX_LOG, "proof batches: n + log_blowup must be at most 17");
+    SR_CHECK(L <= 17, "proof batches: n + log_blowup must be at most 17");
     SR_CHECK(last_log <= FRI_TAIL_MAX_LOG, "proof batches: last layer above 2^10");
     const uint32_t NS = W + 8;  // sampled columns: the trace and the 8 composition halves
     SR_CHECK(NS <= 2048, "proof batches: too many columns");
@@ -278,8 +278,7 @@ static void batch_enqueue(Ctx& c, BatchPlan& P) {
                           L, n);
     }
     DeviceTree tree1{L, P.P0(P.at_tree1), {}}, tree2{L, P.P0(P.at_tree2), {}}, ftree0{L, P.P0(P.at_ftree0), {}};
-    launch_merkle_leaves_dev(c, (const LeafColDev*)P.TB(P.tb_leaf1), P.lp1.segs, W, tree1, K, S);
-    launch_merkle_parents(c, tree1, nullptr, P.P0(P.at_troots), K, S, d_cnt);
+    launch_merkle_tree_dev(c, (const LeafColDev*)P.TB(P.tb_leaf1), P.lp1.segs, W, tree1, P.P0(P.at_troots), K, S, d_cnt);
 
     // mixRoot(main), mixStatement (wide_fibonacci.zig:496-498), composition alpha and its powers
     const uint32_t stw[2] = {n, W};
@@ -296,8 +295,8 @@ static void batch_enqueue(Ctx& c, BatchPlan& P) {
                       CL);
     launch_circle_fft(c, false, (const uint32_t* const*)P.TB(P.tb_cp2), (uint32_t* const*)P.TB(P.tb_lde2), 8 * K, L,
                       n);
-    launch_merkle_leaves_dev(c, (const LeafColDev*)P.TB(P.tb_leaf2), P.lp2.segs, 8, tree2, K, S);
-    launch_merkle_parents(c, tree2, nullptr, P.P0(P.at_troots) + 32, K, S, d_cnt);
+    launch_merkle_tree_dev(c, (const LeafColDev*)P.TB(P.tb_leaf2), P.lp2.segs, 8, tree2, P.P0(P.at_troots) + 32, K, S,
+                           d_cnt);
 
     // mixRoot(composition), OODS point, evaluation factors; sampled values
     uint32_t* d_oods = (uint32_t*)P.P0(P.at_oods);

@@ -160,15 +160,22 @@ struct QuadIo {
     }
 };
 
+// Round r of hash (hlo, hhi) to the board; of the message at byte offset rd from it.
+template <uint32_t N>
+__device__ __forceinline__ void qboard_put_round(uint32_t* board, const QuadIo& io, int r, uint32_t hlo, uint32_t hhi) {
+    *(uint32_t*)((uint8_t*)board + 64 * N * r + io.wr[2 * r]) = hlo;
+    *(uint32_t*)((uint8_t*)board + 64 * N * r + io.wr[2 * r + 1]) = hhi;
+}
+template <uint32_t N>
+__device__ __forceinline__ uint4 qboard_get_round(const uint32_t* board, uint32_t rd, int r) {
+    return *(const uint4*)((const uint8_t*)board + rd + 64 * N * r);
+}
+
 template <uint32_t N>
 __device__ __forceinline__ void qboard_put(uint32_t* board, const QuadIo& io, uint32_t hlo, uint32_t hhi,
                                            uint32_t slot_off = 0) {
-    uint8_t* p = (uint8_t*)(board + 16 * slot_off);
 #pragma unroll
-    for (int r = 0; r < 10; r++) {
-        *(uint32_t*)(p + 64 * N * r + io.wr[2 * r]) = hlo;
-        *(uint32_t*)(p + 64 * N * r + io.wr[2 * r + 1]) = hhi;
-    }
+    for (int r = 0; r < 10; r++) qboard_put_round<N>(board + 16 * slot_off, io, r, hlo, hhi);
 }
 
 // The compression of the message at byte offset rd of the board.
@@ -176,9 +183,8 @@ template <uint32_t N>
 __device__ __forceinline__ void qboard_compress(const QuadLane& L, uint32_t& hlo, uint32_t& hhi,
                                                 const uint32_t* board, uint32_t rd, uint32_t t, bool last) {
     uint4 m[10];
-    const uint8_t* p = (const uint8_t*)board + rd;
 #pragma unroll
-    for (int r = 0; r < 10; r++) m[r] = *(const uint4*)(p + 64 * N * r);
+    for (int r = 0; r < 10; r++) m[r] = qboard_get_round<N>(board, rd, r);
     b2q_compress(L, hlo, hhi, [&](int r) { return m[r]; }, t, last);
 }
 

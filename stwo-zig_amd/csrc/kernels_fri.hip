@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "chan.hpp"
+#include "merkle_leaf.hpp"
 
 namespace sr {
 
@@ -114,10 +115,10 @@ __device__ __forceinline__ void tr_load16(const uint32_t* in, uint32_t m[16]) {
     }
 }
 
-__device__ __forceinline__ void tr_store_quad(uint8_t* __restrict__ g, uint32_t q, uint32_t hlo, uint32_t hhi) {
-    uint32_t* o = (uint32_t*)g;
-    o[q] = hlo;
-    o[4 + q] = hhi;
+// Words q and 4 + q of a hash; `off` = 32 * its index + 4 q.
+__device__ __forceinline__ void tr_store_quad(uint8_t* __restrict__ g, uint32_t off, uint32_t hlo, uint32_t hhi) {
+    *(uint32_t*)(g + off) = hlo;
+    *(uint32_t*)(g + off + 16) = hhi;
 }
 
 __device__ __forceinline__ void tr_put_lane(uint32_t* lds, uint8_t* __restrict__ g, const uint32_t h[8]) {
@@ -142,33 +143,50 @@ struct TrQuad {
     }
 };
 
-// Address of hash `first` of tree level `lev`.
-__device__ __forceinline__ uint8_t* tr_at(uint8_t* tree, uint32_t lev, uint64_t first) {
-    return tree + ((((uint64_t)1 << lev) - 1) + first) * 32;
-}
-
 // The levels of c, c/2, ..., 1 parents by quads; the 2c children are on the board, written by
 // quads 0 .. 2c - 1.  Level `lev` has c parents of this workgroup, from parent blk * c on.  The
-// root ends as (rlo, rhi) = words (q, 4 + q) in quads 0 and 1 (the channel step takes it from
-// both).  Waves other than the first leave once the first is alone with the rest.
+// root ends as (rlo, rhi) = words (q, 4 + q) in every quad of the first wave; the other waves
+// leave once the first is alone with the rest.  There its quads all compress, also those beyond
+// the level (on words that nothing valid comes from: quad i writes slot i / 2, and only slots
+// below the next level's count are read for a result): what a level costs is one wave's
+// instructions, and masks and branches are among them.
 __device__ __forceinline__ void tr_quad_levels(const TrQuad& Q, uint32_t* board, uint32_t c, uint8_t* tree,
-                                               uint32_t lev, uint64_t blk, uint32_t& rlo, uint32_t& rhi) {
-    const uint32_t p = Q.t >> 2;
-    for (;; c >>= 1, lev--) {
-        if (2 * c > TR_WAVE_MAX) __syncthreads();
-        else if (Q.t >= 64) return;
-        else qboard_wave_fence();
-        if (p < c || (c == 1 && p == 1)) {
-            rlo = Q.nlo;
-            rhi = Q.nhi;
-            qboard_compress<TR_BOARD>(Q.L, rlo, rhi, board, c == 1 ? 16 * Q.q : Q.io.rd, 128, true);
-        }
+                                               uint32_t lev, uint32_t blk, uint32_t& rlo, uint32_t& rhi) {
+    const uint32_t p = Q.t >> 2, wave = __builtin_amdgcn_readfirstlane(Q.t >> 6);
+    const uint32_t node = 32 * p + 4 * Q.q;
+    uint32_t at = (1u << lev) - 1 + blk * c;  // this workgroup's first parent among the tree's hashes
+    for (; 2 * c > TR_WAVE_MAX; c >>= 1, at >>= 1) {
+        __syncthreads();
+        rlo = Q.nlo;
+        rhi = Q.nhi;
+        if (TR_WAVE_MAX * wave < c)
+            qboard_compress<TR_BOARD>(Q.L, rlo, rhi, board, Q.io.rd, 128, true);
         if (c > TR_WAVE_MAX) __syncthreads();  // every message is read
-        if (p < c) {
-            if (c > 1) qboard_put<TR_BOARD>(board, Q.io, rlo, rhi);
-            tr_store_quad(tr_at(tree, lev, blk * c) + 32 * p, Q.q, rlo, rhi);
+        if (TR_WAVE_MAX * wave < c) {
+            qboard_put<TR_BOARD>(board, Q.io, rlo, rhi);
+            tr_store_quad(tree, 32 * at + node, rlo, rhi);
         }
+    }
+    if (wave) return;
+    uint32_t rd = c == 1 ? 16 * Q.q : Q.io.rd;
+    uint4 m[10];
+    qboard_wave_fence();
+#pragma unroll
+    for (int r = 0; r < 10; r++) m[r] = qboard_get_round<TR_BOARD>(board, rd, r);
+    for (;; at >>= 1) {
+        rlo = Q.nlo;
+        rhi = Q.nhi;
+        b2q_compress(Q.L, rlo, rhi, [&](int r) { return m[r]; }, 128, true);
+        if (p < c) tr_store_quad(tree, 32 * at + node, rlo, rhi);
         if (c == 1) return;
+        c >>= 1;
+        rd = c == 1 ? 16 * Q.q : rd;
+#pragma unroll
+        for (int r = 0; r < 10; r++) {
+            qboard_put_round<TR_BOARD>(board, Q.io, r, rlo, rhi);
+            qboard_wave_fence();
+            m[r] = qboard_get_round<TR_BOARD>(board, rd, r);
+        }
     }
 }
 
@@ -177,12 +195,12 @@ __device__ __forceinline__ void tr_quad_levels(const TrQuad& Q, uint32_t* board,
 // the levels on the board, which may overlap that level's inputs.
 template <uint32_t T>
 __device__ __forceinline__ void tr_levels(const TrQuad& Q, uint32_t* lds, bool on_board, uint32_t c, uint8_t* tree,
-                                          uint32_t lev, uint64_t blk, const B2State& seed, uint32_t& rlo,
+                                          uint32_t lev, uint32_t blk, const B2State& seed, uint32_t& rlo,
                                           uint32_t& rhi) {
     if (!on_board) {
         uint32_t *in = lds, *out = lds + TR_PLAIN_A;
         for (; c > TR_QUAD_MAX; c >>= 1, lev--) {
-            uint8_t* g = tr_at(tree, lev, blk * c);
+            uint8_t* g = tree + 32ull * ((1u << lev) - 1 + blk * c);
             for (uint32_t p = Q.t; p < c; p += T) {
                 uint32_t m[16], h[8];
                 tr_load16(in + 16 * p, m);
@@ -198,25 +216,22 @@ __device__ __forceinline__ void tr_levels(const TrQuad& Q, uint32_t* lds, bool o
         }
         constexpr uint32_t STEP = T / 4, IT = (TR_QUAD_MAX + STEP - 1) / STEP;
         uint32_t lo[IT], hi[IT];
-#pragma unroll
-        for (uint32_t k = 0; k < IT; k++) {
-            lo[k] = Q.nlo;
-            hi[k] = Q.nhi;
-        }
+        uint8_t* g = tree + 32ull * ((1u << lev) - 1 + blk * c);
         // one copy of the compression's code
 #pragma unroll 1
         for (uint32_t k = 0; k < IT; k++) {
             const uint32_t p = (Q.t >> 2) + k * STEP;
-            if (p < c || (c == 1 && p == 1)) {
-                uint32_t m[16], hlo = Q.nlo, hhi = Q.nhi;
+            uint32_t hlo = Q.nlo, hhi = Q.nhi;
+            if (p < c || (c == 1 && Q.t < 64 && k == 0)) {
+                uint32_t m[16];
                 tr_load16(in + (c == 1 ? 0 : 16 * p), m);
                 b2_compress_quad(Q.L, hlo, hhi, m, 128, true);
-                if (p < c) tr_store_quad(tr_at(tree, lev, blk * c) + 32 * p, Q.q, hlo, hhi);
+                if (p < c) tr_store_quad(g, 32 * p + 4 * Q.q, hlo, hhi);
+            }
 #pragma unroll
-                for (uint32_t i = 0; i < IT; i++) {
-                    lo[i] = i == k ? hlo : lo[i];
-                    hi[i] = i == k ? hhi : hi[i];
-                }
+            for (uint32_t i = 0; i < IT; i++) {
+                lo[i] = i == k ? hlo : lo[i];
+                hi[i] = i == k ? hhi : hi[i];
             }
         }
         rlo = lo[0];
@@ -266,28 +281,33 @@ __device__ __forceinline__ qm31 tr_fold_at(const FriLayerArgs& a, uint64_t i, qm
     }
 }
 
-// The channel in LDS: two one-slot boards, the message of mixRoot (digest || root) and that of
-// drawSecureFelt (digest || draw counter || zeros).  All threads; the caller's barrier ends it.
+// The channel beside the levels: the digest as words (q, 4 + q) in every quad of the first wave,
+// the draws since the last mix, the last drawn element; in LDS two one-slot boards, the message of
+// mixRoot (digest || root) and that of drawSecureFelt (digest || draw counter || zeros).
+struct TrChan {
+    uint32_t dlo, dhi, n_draws;
+    qm31 alpha;
+};
+
+// All threads; the caller's barrier ends it.
 template <uint32_t T>
-__device__ __forceinline__ void tr_chan_init(const TrQuad& Q, uint32_t* chan, const DevChannel* ch) {
+__device__ __forceinline__ TrChan tr_chan_init(const TrQuad& Q, uint32_t* chan, const DevChannel* ch) {
     if (Q.t >= 64) {
         for (uint32_t i = Q.t - 64; i < 160; i += T - 64) chan[160 + i] = 0;
-    } else if (Q.t < 4) {
-        qboard_put<1>(chan, Q.io, ch->digest[Q.q], ch->digest[4 + Q.q]);
     }
+    return TrChan{ch->digest[Q.q], ch->digest[4 + Q.q], 0, qzero()};
 }
 
-// Channel step on a root held by quads 0 and 1 (the threads that run it) as (rlo, rhi)
-// (MerkleChannel.mixRoot then drawSecureFelt, as chan_mix_root_draw_quad): updates the LDS
-// messages and the DevChannel, copies the root to root_out.
-__device__ __forceinline__ qm31 tr_chan_step(const TrQuad& Q, uint32_t* chan, uint32_t rlo, uint32_t rhi,
-                                             DevChannel* __restrict__ ch, uint32_t* __restrict__ root_out) {
+// Channel step on a root held by every quad of the first wave, which runs it, as (rlo, rhi)
+// (MerkleChannel.mixRoot then drawSecureFelt, as chan_mix_root_draw_quad).
+__device__ __forceinline__ void tr_chan_step(const TrQuad& Q, uint32_t* chan, uint32_t rlo, uint32_t rhi, TrChan& C,
+                                             DevChannel* __restrict__ ch) {
     const QuadLane& L = Q.L;
     const uint32_t ilo = L.sel(SR_B2_IV0 ^ 0x01010020u, SR_B2_IV1, SR_B2_IV2, SR_B2_IV3);
     const uint32_t ihi = L.sel(SR_B2_IV4, SR_B2_IV5, SR_B2_IV6, SR_B2_IV7);
     uint32_t *const mix = chan, *const draw = chan + 160;
-    if (Q.t >= 4) qboard_put<1>(mix, Q.io, rlo, rhi);
-    uint32_t dlo = 0, dhi = 0;
+    // quad 0 writes the first half of a message, quad 1 the second
+    if (Q.t < 8) qboard_put<1>(mix, Q.io, Q.t < 4 ? C.dlo : rlo, Q.t < 4 ? C.dhi : rhi);
     // compression 0 is the mix, the others are draws (more than one with probability ~2^-28)
 #pragma unroll 1
     for (uint32_t k = 0; k <= 64; k++) {
@@ -295,44 +315,48 @@ __device__ __forceinline__ qm31 tr_chan_step(const TrQuad& Q, uint32_t* chan, ui
         uint32_t hlo = ilo, hhi = ihi;
         qboard_compress<1>(L, hlo, hhi, k ? draw : mix, 16 * Q.q, k ? 37 : 64, true);
         if (k == 0) {
-            dlo = hlo;
-            dhi = hhi;
-            if (Q.t < 4) qboard_put<1>(draw, Q.io, dlo, dhi);
+            C.dlo = hlo;
+            C.dhi = hhi;
+            if (Q.t < 4) qboard_put<1>(draw, Q.io, hlo, hhi);
             continue;
         }
         uint32_t bad = (hlo >= 2u * P || hhi >= 2u * P) ? 1u : 0u;
         bad |= quad_perm<QP_ROT1>(bad);
-        bad |= quad_perm<QP_ROT2>(bad);  // OR over the quad (the same in both)
-        // message word 8, the draw counter (the first word of the second half): the next one, or
-        // zero again for the next step
-        if ((bad || k > 1) && Q.t == 4) {
+        bad |= quad_perm<QP_ROT2>(bad);  // OR over the quad (the same in all)
+        bad = __builtin_amdgcn_readfirstlane(bad);
+        if (bad || k > 1) {
+            // message word 8, the draw counter (the first word of the second half): the next one,
+            // or zero again for the next step
+            if (Q.t == 4) {
 #pragma unroll
-            for (int r = 0; r < 10; r++) *(uint32_t*)((uint8_t*)draw + 64 * r + Q.io.wr[2 * r]) = bad ? k : 0u;
-        }
-        if (bad) continue;
-        const qm31 a = {{mred64(quad_bcast<0>(hlo)), mred64(quad_bcast<1>(hlo))},
-                        {mred64(quad_bcast<2>(hlo)), mred64(quad_bcast<3>(hlo))}};
-        if (Q.t < 4) {
-            qboard_put<1>(mix, Q.io, dlo, dhi);
-            if (root_out) tr_store_quad((uint8_t*)root_out, Q.q, rlo, rhi);
-            ch->digest[Q.q] = dlo;
-            ch->digest[4 + Q.q] = dhi;
-            if (Q.q == 0) {
-                ch->n_draws = k;
-                qstore(a, ch->alpha);
-                qstore(qsqr(a), ch->alpha2);
+                for (int r = 0; r < 10; r++) *(uint32_t*)((uint8_t*)draw + 64 * r + Q.io.wr[2 * r]) = bad ? k : 0u;
             }
+            if (bad) continue;
         }
-        return a;
+        C.n_draws = k;
+        C.alpha = {{mred64(quad_bcast<0>(hlo)), mred64(quad_bcast<1>(hlo))},
+                   {mred64(quad_bcast<2>(hlo)), mred64(quad_bcast<3>(hlo))}};
+        return;
     }
     if (Q.t == 0) ch->status = 1;
-    return qzero();
+}
+
+// The state of the first wave's channel to the DevChannel.
+__device__ __forceinline__ void tr_chan_store(const TrQuad& Q, const TrChan& C, DevChannel* __restrict__ ch) {
+    if (Q.t >= 4) return;
+    ch->digest[Q.q] = C.dlo;
+    ch->digest[4 + Q.q] = C.dhi;
+    if (Q.q == 0) {
+        ch->n_draws = C.n_draws;
+        qstore(C.alpha, ch->alpha);
+        qstore(qsqr(C.alpha), ch->alpha2);
+    }
 }
 
 // One tree (or its top levels) in one launch.  Workgroup b owns the 2^s hashes
 // [b 2^s, (b+1) 2^s) of level k0: it produces them (SRC = FRI_SRC_LINE / FRI_SRC_CIRCLE:
 // fold the previous layer with the alpha in `ch`, store the folded value and hash it as a
-// leaf) or loads them (FRI_SRC_HASHES), then reduces them to its subtree root at level
+// leaf; FRI_SRC_COLUMNS: hash the rows of a tree's columns) or loads them (FRI_SRC_HASHES), then reduces them to its subtree root at level
 // k0 - s.  The last workgroup to finish (split completion counters; the subtree roots are
 // exchanged through device-coherent stores and loads, so no workgroup writes back its L2)
 // reduces the 2^(k0-s) subtree roots to the root and, with `ch`, runs the channel step on
@@ -371,6 +395,40 @@ __global__ __launch_bounds__(TL_THREADS) void tree_layer_kernel(FriLayerArgs a0)
             *(uint4*)&lds[8 * p] = x;
             *(uint4*)&lds[8 * p + 4] = y;
         }
+    } else if constexpr (SRC == FRI_SRC_COLUMNS) {
+        const uint64_t boff = (uint64_t)blockIdx.y * a.bstride;
+        const uint32_t nblk = (a.n_cols + 15) >> 4;
+        boards = n1 <= TR_QUAD_MAX;
+        if (boards) {
+#pragma unroll 1
+            for (uint32_t k = 0; k < TR_QUAD_MAX / (TL_THREADS / 4); k++) {
+                const uint32_t p = (t >> 2) + k * (TL_THREADS / 4);
+                if (p >= n1) break;
+                const uint32_t voff = (uint32_t)(base + p) << 2;
+                uint32_t hlo = Q.L.sel(a.leaf_seed.h[0], a.leaf_seed.h[1], a.leaf_seed.h[2], a.leaf_seed.h[3]);
+                uint32_t hhi = Q.L.sel(a.leaf_seed.h[4], a.leaf_seed.h[5], a.leaf_seed.h[6], a.leaf_seed.h[7]);
+                uint32_t m[16], nx[16];
+                leaf_block_load_ident<true>(a.cols, voff, m, boff);
+#pragma unroll 1
+                for (uint32_t b = 0; b < nblk; b++) {
+                    const bool lst = b + 1 == nblk;
+                    if (!lst) leaf_block_load_ident<true>(a.cols + 16 * (b + 1), voff, nx, boff);
+                    b2_compress_quad(Q.L, hlo, hhi, m, 64 + (lst ? 4 * a.n_cols : 64 * (b + 1)), lst);
+#pragma unroll
+                    for (int w = 0; w < 16; w++) m[w] = nx[w];
+                }
+                qboard_put<TR_BOARD>(lds, Q.io, hlo, hhi, k * (TL_THREADS / 8));
+                tr_store_quad(lev_k0 + base * 32, 32 * p + 4 * q, hlo, hhi);
+            }
+        } else {
+            for (uint32_t p = t; p < n1; p += TL_THREADS) {
+                uint32_t h[8];
+#pragma unroll
+                for (int k = 0; k < 8; k++) h[k] = a.leaf_seed.h[k];
+                leaf_hash_ident(a.cols, 0, nblk, a.n_cols, (uint32_t)(base + p) << 2, boff, h);
+                tr_put_lane(lds + 8 * p, lev_k0 + (base + p) * 32, h);
+            }
+        }
     } else {
         const qm31 alpha = qload(a.ch->alpha);
         boards = n1 <= TR_QUAD_MAX;
@@ -384,7 +442,7 @@ __global__ __launch_bounds__(TL_THREADS) void tree_layer_kernel(FriLayerArgs a0)
                     uint32_t hlo, hhi;
                     tr_leaf_quad(Q.L, a.leaf_seed, r, hlo, hhi);
                     qboard_put<TR_BOARD>(lds, Q.io, hlo, hhi, k * (TL_THREADS / 8));
-                    tr_store_quad(lev_k0 + (base + p) * 32, q, hlo, hhi);
+                    tr_store_quad(lev_k0 + base * 32, 32 * p + 4 * q, hlo, hhi);
                 }
             }
         } else {
@@ -401,9 +459,10 @@ __global__ __launch_bounds__(TL_THREADS) void tree_layer_kernel(FriLayerArgs a0)
     // nothing of the top pass is kept for the first one: the channel's boards are written by the
     // workgroup that reaches the root
     uint32_t c = n1 >> 1, lev = a.k0 - 1;
-    uint64_t blk = blockIdx.x;
+    uint32_t blk = blockIdx.x;
+    TrChan C{};
     for (bool top = nb == 1;; top = true) {
-        if (top && a.ch) tr_chan_init<TL_THREADS>(Q, chan, a.ch);
+        if (top && a.ch) C = tr_chan_init<TL_THREADS>(Q, chan, a.ch);
         if (!boards || top) __syncthreads();
         tr_levels<TL_THREADS>(Q, lds, boards, c, a.tree, lev, blk, a.node_seed, rlo, rhi);
         if (top) break;
@@ -442,10 +501,11 @@ __global__ __launch_bounds__(TL_THREADS) void tree_layer_kernel(FriLayerArgs a0)
         lev = a.k0 - a.s - 1;
         blk = 0;
     }
+    if (t >= 64) return;
+    if (t < 4 && a.root_out) tr_store_quad((uint8_t*)a.root_out, 4 * q, rlo, rhi);
     if (a.ch) {
-        if (t < 8) (void)tr_chan_step(Q, chan, rlo, rhi, a.ch, a.root_out);
-    } else if (t < 4 && a.root_out) {
-        tr_store_quad((uint8_t*)a.root_out, q, rlo, rhi);
+        tr_chan_step(Q, chan, rlo, rhi, C, a.ch);
+        tr_chan_store(Q, C, a.ch);
     }
 }
 
@@ -474,54 +534,62 @@ __global__ __launch_bounds__(TAIL_THREADS) void fri_tail_kernel(const FriTailArg
     const uint32_t t = threadIdx.x, q = t & 3;
     const TrQuad Q(t, node_seed);
     uint32_t l = a.top_log;
-    qm31 alpha = qload(ch->alpha);
-    tr_chan_init<TAIL_THREADS>(Q, chan, ch);
+    TrChan C = tr_chan_init<TAIL_THREADS>(Q, chan, ch);
+    C.alpha = qload(ch->alpha);
     // This thread's value k of a layer of n values: its quad's on narrow layers, else its lane's.
-    // The inverse x of the next layer's are loaded while this one's tree is hashed.
+    // The next layer's pointers and inverse x are loaded while this one's tree is hashed.
     uint32_t inv[PER];
+    uint4* line;
+    uint8_t* tree;
+    uint32_t* root;
     const auto value = [&](uint32_t n, uint32_t k) {
         return n <= TR_QUAD_MAX ? (k ? n : t >> 2) : t + k * TAIL_THREADS;
     };
-    const auto load_inv = [&](uint32_t log) {
-        const uint32_t n = 1u << (log - 1);
-        const uint32_t* inv_x = a.itw_half - ((size_t)1 << log);
+    const auto load_layer = [&](uint32_t log) {
+        const uint32_t n = 1u << log;
+        const uint32_t* inv_x = a.itw_half - 2 * (size_t)n;
 #pragma unroll
         for (uint32_t k = 0; k < PER; k++) inv[k] = value(n, k) < n ? inv_x[value(n, k)] : 0u;
+        line = at(a.lines[log]);
+        tree = at(a.trees[log]);
+        root = a.roots[log] ? at(a.roots[log]) : nullptr;
+        asm volatile("" : "+s"(line), "+s"(tree), "+s"(root));  // here, not where they are used
     };
-    load_inv(l);
+    load_layer(l - 1);
     __syncthreads();
+    const uint4* __restrict__ src = at(a.lines[l]);
     bool first = true;
     for (;;) {
-        const uint32_t n = 1u << (l - 1);
+        l--;
+        const uint32_t n = 1u << l;
         const bool quads = n <= TR_QUAD_MAX;
         qm31 r[PER];
 #pragma unroll
         for (uint32_t k = 0; k < PER; k++) {
             const uint32_t p = value(n, k);
             if (p < n) {
-                const uint4* __restrict__ src = at(a.lines[l]);
                 const uint4 x = first ? src[2 * p] : vs[2 * p];
                 const uint4 y = first ? src[2 * p + 1] : vs[2 * p + 1];
-                r[k] = tr_fold(x, y, alpha, inv[k]);
+                r[k] = tr_fold(x, y, C.alpha, inv[k]);
             }
         }
         first = false;
         if (n <= TR_WAVE_MAX) qboard_wave_fence();
         else __syncthreads();
-        l--;
 #pragma unroll
         for (uint32_t k = 0; k < PER; k++) {
             const uint32_t p = value(n, k);
             if (p < n && (!quads || q == 0)) {
                 const uint4 rv = make_uint4(r[k].c0.a, r[k].c0.b, r[k].c1.a, r[k].c1.b);
                 vs[p] = rv;
-                at(a.lines[l])[p] = rv;
+                line[p] = rv;
             }
         }
         if (l == a.last_log) break;
-        load_inv(l);
-        uint8_t* tree = at(a.trees[l]);
-        uint8_t* leaves = tree + (((size_t)1 << l) - 1) * 32;
+        const uint64_t leaves = 32ull * (n - 1);
+        uint8_t* const tr = tree;
+        uint32_t* const ro = root;
+        load_layer(l - 1);
         uint32_t rlo = 0, rhi = 0;
         if (quads) {
             const uint32_t p = t >> 2;
@@ -529,7 +597,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void fri_tail_kernel(const FriTailArg
                 uint32_t hlo, hhi;
                 tr_leaf_quad(Q.L, leaf_seed, r[0], hlo, hhi);
                 qboard_put<TR_BOARD>(lds, Q.io, hlo, hhi);
-                tr_store_quad(leaves + (size_t)p * 32, q, hlo, hhi);
+                tr_store_quad(tr + leaves, 32 * p + 4 * q, hlo, hhi);
             }
         } else {
 #pragma unroll
@@ -538,22 +606,29 @@ __global__ __launch_bounds__(TAIL_THREADS) void fri_tail_kernel(const FriTailArg
                 if (p < n) {
                     uint32_t h[8];
                     tr_leaf_lane(leaf_seed, r[k], h);
-                    tr_put_lane(lds + 8 * p, leaves + (size_t)p * 32, h);
+                    tr_put_lane(lds + 8 * p, tr + leaves + 32 * p, h);
                 }
             }
             __syncthreads();
         }
-        tr_levels<TAIL_THREADS>(Q, lds, quads, n >> 1, tree, l - 1, 0, node_seed, rlo, rhi);
-        if (t < 8) {
-            alpha = tr_chan_step(Q, chan, rlo, rhi, ch, a.roots[l] ? at(a.roots[l]) : nullptr);
-            if (t == 0) qstore(alpha, sa);
+        tr_levels<TAIL_THREADS>(Q, lds, quads, n >> 1, tr, l - 1, 0, node_seed, rlo, rhi);
+        // the next layer folds in the first wave alone if it has at most 16 values
+        const bool alone = n <= 2 * TR_WAVE_MAX;
+        if (t < 64) {
+            if (t < 4 && ro) tr_store_quad((uint8_t*)ro, 4 * q, rlo, rhi);
+            tr_chan_step(Q, chan, rlo, rhi, C, ch);
+            if (t == 0 && !alone) qstore(C.alpha, sa);
+        } else if (alone) {
+            return;
         }
-        // the next layer folds in the first wave only if it has at most 16 values
-        if (n > 2 * TR_WAVE_MAX) __syncthreads();
-        else if (t >= 64) return;
-        else qboard_wave_fence();
-        alpha = qload(sa);
+        if (alone) {
+            qboard_wave_fence();
+        } else {
+            __syncthreads();
+            if (t >= 64) C.alpha = qload(sa);
+        }
     }
+    if (t < 64 && C.n_draws) tr_chan_store(Q, C, ch);
 }
 
 // Hashes per workgroup (log) for a tree reduction from level k0: the whole tree in one
@@ -598,11 +673,26 @@ void launch_tree_top(Ctx& c, DeviceTree& t, uint32_t k0, DevChannel* d_ch, uint8
                                       32.0 * (double)((2ull << k0) - 1), batch, bstride, d_cnt);
 }
 
+void launch_tree_from_columns(Ctx& c, const LeafColDev* d_tab, uint32_t n_cols, DeviceTree& t, uint8_t* d_root_out,
+                              uint32_t batch, uint64_t bstride, uint32_t* d_cnt) {
+    SR_CHECK(d_tab && n_cols >= 1, "tree: no columns");
+    FriLayerArgs a{};
+    a.cols = d_tab;
+    a.n_cols = n_cols;
+    a.tree = t.layers;
+    a.k0 = t.max_log;
+    a.root_out = (uint32_t*)d_root_out;
+    const double n = (double)(1ull << t.max_log);
+    launch_tree_layer<FRI_SRC_COLUMNS>(c, a,
+                                       "merkle_tree L=" + std::to_string(t.max_log) + " cols=" + std::to_string(n_cols),
+                                       4.0 * n_cols * n + 32.0 * (2.0 * n - 1.0), batch, bstride, d_cnt);
+}
+
 void launch_fri_commit_line(Ctx& c, const uint32_t* d_src, uint32_t log_src, uint32_t* d_dst, DeviceTree& t,
                             DevChannel* d_ch, uint8_t* d_root_out, uint32_t batch, uint64_t bstride, uint32_t* d_cnt) {
     const uint32_t l = log_src - 1;
     SR_CHECK(log_src >= 1 && t.max_log == l && d_ch, "fri commit: layer shape");
-    if (l == 0 || l > TREE_LAYER_MAX_LOG) {
+    if (l == 0 || l > FRI_LAYER_MAX_LOG) {
         SR_CHECK(batch == 1, "fri commit: batches of layers above 2^16");
         launch_fold_line(c, d_src, log_src, qzero(), d_dst, t.layer(l), d_ch);
         launch_merkle_parents(c, t, d_ch, d_root_out);
@@ -627,7 +717,7 @@ void launch_fri_commit_circle(Ctx& c, const uint32_t* const* coords, uint32_t lo
                               uint32_t* d_cnt) {
     const uint32_t l = log_src - 1;
     SR_CHECK(log_src >= 1 && t.max_log == l && d_ch, "fri commit: layer shape");
-    if (l == 0 || l > TREE_LAYER_MAX_LOG) {
+    if (l == 0 || l > FRI_LAYER_MAX_LOG) {
         SR_CHECK(batch == 1, "fri commit: batches of layers above 2^16");
         launch_fold_circle_into_line(c, coords, log_src, qzero(), d_dst, false, t.layer(l), d_ch);
         launch_merkle_parents(c, t, d_ch, d_root_out);

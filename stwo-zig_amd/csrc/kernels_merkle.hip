@@ -15,17 +15,17 @@
 // 2^L times.  The result is the same leaf hash.
 //
 // Parents (layers.zig:99-140; blake2_merkle.zig:112-154): node = Blake2s(
-// "node"+0^60 || left || right), one compression from the node seed.  One
-// launch builds up to 10 levels: each thread hashes four children from HBM
-// into two parents and their parent in registers, then the block halves the
-// level in LDS, writing every level; levels of at most 64 nodes use one quad of
-// lanes per compression.  The last 16 or fewer levels are one tree-layer launch
-// (kernels_fri.hip) whose workgroups reduce up to 2^10 hashes each and whose last
-// workgroup reduces their roots.  A 2^21-leaf tree takes two launches instead of 21.
+// "node"+0^60 || left || right), one compression from the node seed.  The wide levels
+// take a launch per three (parent_levels): each thread hashes four children from HBM into two parents and
+// their parent in registers, then the block halves the level in LDS.  The last 18 or fewer
+// levels are one tree-layer launch (kernels_fri.hip) whose workgroups reduce up to 2^10 hashes
+// each and whose last workgroup reduces their roots; up to 2^19 leaves of equal columns that launch
+// hashes the leaves too.
 #include <algorithm>
 #include <vector>
 
 #include "chan.hpp"
+#include "merkle_leaf.hpp"
 
 namespace sr {
 
@@ -35,30 +35,6 @@ __device__ __forceinline__ void store_hash(uint8_t* __restrict__ out, uint64_t i
     uint4* o = (uint4*)(out + i * 32);
     o[0] = make_uint4(h[0], h[1], h[2], h[3]);
     o[1] = make_uint4(h[4], h[5], h[6], h[7]);
-}
-
-// boff: byte offset of the proof's columns in a batch (0 for one tree).
-__device__ __forceinline__ void leaf_block_load(const LeafColDev* __restrict__ cd, uint32_t p, uint32_t m[16],
-                                                uint64_t boff) {
-#pragma unroll
-    for (int w = 0; w < 16; w++) {
-        const LeafColDev d = cd[w];
-        m[w] = ((gcu32*)((const uint8_t*)d.col + boff))[((p >> d.shift) << 1) + (p & 1)] & d.mask;
-    }
-}
-
-// The same for a segment whose columns all have the segment's size (lift(p) = p): every
-// word is the column pointer (uniform) plus the lane's byte offset p * 4 (rows < 2^30), and
-// the padding mask applies only to a padded last block (MASKED).
-template <bool MASKED>
-__device__ __forceinline__ void leaf_block_load_ident(const LeafColDev* __restrict__ cd, uint32_t voff,
-                                                      uint32_t m[16], uint64_t boff) {
-#pragma unroll
-    for (int w = 0; w < 16; w++) {
-        const LeafColDev d = cd[w];
-        const uint32_t x = *(gcu32*)((const SR_GLOBAL uint8_t*)d.col + boff + voff);
-        m[w] = MASKED ? (x & d.mask) : x;
-    }
 }
 
 // One state per lane over blocks [blk0, blk0 + nblk) of a segment at `level`: the
@@ -91,26 +67,7 @@ __global__ __launch_bounds__(MK_THREADS) void merkle_leaves_kernel(const LeafCol
     const uint32_t nblocks_total = (n_cols + 15) >> 4;
     const uint32_t blk_end = blk0 + nblk;
     if constexpr (IDENT) {
-        // blocks of 16 real columns, then at most one padded block (the last of the leaf)
-        const uint32_t full_end = ((n_cols & 15) && blk_end == nblocks_total) ? blk_end - 1 : blk_end;
-        const uint32_t voff = p << 2;
-        uint32_t a[16], b[16];
-        uint32_t blk = blk0;
-        if (blk < full_end) leaf_block_load_ident<false>(cols + 16 * blk, voff, a, boff);
-        for (; blk + 1 < full_end; blk += 2) {
-            leaf_block_load_ident<false>(cols + 16 * (blk + 1), voff, b, boff);
-            b2_compress(h, a, 64 + 64 * (blk + 1), blk + 1 == nblocks_total);
-            if (blk + 2 < full_end) leaf_block_load_ident<false>(cols + 16 * (blk + 2), voff, a, boff);
-            b2_compress(h, b, 64 + 64 * (blk + 2), blk + 2 == nblocks_total);
-        }
-        if (blk < full_end) {
-            b2_compress(h, a, 64 + 64 * (blk + 1), blk + 1 == nblocks_total);
-            blk++;
-        }
-        if (blk < blk_end) {
-            leaf_block_load_ident<true>(cols + 16 * blk, voff, a, boff);
-            b2_compress(h, a, 64 + 4 * n_cols, true);
-        }
+        leaf_hash_ident(cols, blk0, blk_end, n_cols, p << 2, boff, h);
     } else {
         uint32_t cur[16];
         leaf_block_load(cols + 16 * blk0, p, cur, boff);
@@ -190,13 +147,14 @@ __global__ __launch_bounds__(MK_THREADS) void merkle_leaves_qm31_kernel(const ui
     store_hash(leaves, p, h);
 }
 
-// Builds `levels` (2..10) parent levels below layer k.  Block b covers the
-// 2^levels * ... children [b*4T, (b+1)*4T) of layer k for T = 2^(levels-2)
-// threads: every thread hashes two parents of level k-1 from four children
-// (two independent compressions) and their parent of level k-2 in registers,
-// so the first two levels keep every lane busy; the remaining levels halve in
-// LDS.  levels == 1 uses one thread per parent.
-constexpr int MP_THREADS = 256;
+// Levels k-1 .. k-levels (2..10) of a tree of at least 2^10 hashes at level k.  A block takes 1024
+// of them: every thread hashes two parents of level k-1 from four children (two independent
+// compressions) and their parent of level k-2 in registers; the remaining levels halve in LDS,
+// by one lane per compression while that fills whole waves, then by quads.  The kernel is bound
+// by the instructions of its compressions, and every level after the first two leaves more of
+// the block's lanes idle: from 2^24 hashes, ten levels take 591 us for 2^24 compressions, four
+// 493, three 445 for 7/8 of them; the leaves' 2^24 would take 500 at the rate of a 100-column tree.
+constexpr uint32_t MP_THREADS = 256;
 __device__ __forceinline__ void node_hash(const B2State& seed, const uint32_t* l, const uint32_t* r, uint32_t h[8]) {
     uint32_t m[16];
 #pragma unroll
@@ -209,28 +167,14 @@ __device__ __forceinline__ void node_hash(const B2State& seed, const uint32_t* l
     b2_compress(h, m, 128, true);
 }
 
-// Levels k-1 .. k-levels of a tree: block b reduces its 2^levels hashes of level k.
 __global__ __launch_bounds__(MP_THREADS) void merkle_parents_kernel(uint8_t* __restrict__ tree, uint32_t k,
                                                                     uint32_t levels, B2State seed, uint64_t bstride) {
     __shared__ uint32_t sh[MP_THREADS * 8];
     const uint32_t t = threadIdx.x;
     tree += (uint64_t)blockIdx.y * bstride;  // tree blockIdx.y of a batch
     const uint8_t* child = tree + (((uint64_t)1 << k) - 1) * 32;
-    if (levels == 1) {
-        uint64_t i = (uint64_t)blockIdx.x * MP_THREADS + t;
-        if (i >= (1ull << (k - 1))) return;
-        const uint4* c4 = (const uint4*)(child + i * 64);
-        uint4 a = c4[0], b = c4[1], c = c4[2], d = c4[3];
-        uint32_t l[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, r[8] = {c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w};
-        uint32_t h[8];
-        node_hash(seed, l, r, h);
-        store_hash(tree + (((uint64_t)1 << (k - 1)) - 1) * 32, i, h);
-        return;
-    }
-    const uint32_t T = 1u << (levels - 2);  // threads with work (<= 256)
-    uint64_t g = (uint64_t)blockIdx.x * T + t;  // index at level k-2
-    uint32_t h2[8];
-    if (t < T) {
+    const uint64_t g = (uint64_t)blockIdx.x * MP_THREADS + t;  // index at level k-2
+    {
         const uint4* c4 = (const uint4*)(child + g * 128);
         uint32_t c[32];
 #pragma unroll
@@ -241,7 +185,7 @@ __global__ __launch_bounds__(MP_THREADS) void merkle_parents_kernel(uint8_t* __r
             c[4 * q + 2] = v.z;
             c[4 * q + 3] = v.w;
         }
-        uint32_t p0[8], p1[8];
+        uint32_t p0[8], p1[8], h2[8];
         node_hash(seed, c, c + 8, p0);
         node_hash(seed, c + 16, c + 24, p1);
         uint8_t* l1 = tree + (((uint64_t)1 << (k - 1)) - 1) * 32;
@@ -252,8 +196,8 @@ __global__ __launch_bounds__(MP_THREADS) void merkle_parents_kernel(uint8_t* __r
 #pragma unroll
         for (int i = 0; i < 8; i++) sh[t * 8 + i] = h2[i];
     }
-    uint32_t count = T, level = k - 2;
-    uint64_t first = (uint64_t)blockIdx.x * T;
+    uint32_t count = MP_THREADS, level = k - 2;
+    uint64_t first = (uint64_t)blockIdx.x * MP_THREADS;
     const uint32_t q = t & 3, j = t >> 2;
     const QuadLane L(q);
     for (uint32_t lv = 2; lv < levels; lv++) {
@@ -262,7 +206,7 @@ __global__ __launch_bounds__(MP_THREADS) void merkle_parents_kernel(uint8_t* __r
         level--;
         first >>= 1;
         uint8_t* out = tree + (((uint64_t)1 << level) - 1) * 32;
-        if (count > blockDim.x / 4) {
+        if (count >= 64) {
             uint32_t h[8];
             if (t < count) node_hash(seed, &sh[t * 16], &sh[t * 16 + 8], h);
             __syncthreads();
@@ -398,13 +342,6 @@ void launch_merkle_leaves_dev(Ctx& c, const LeafColDev* d_tab, const std::vector
     }
 }
 
-void launch_merkle_leaves(Ctx& c, const uint32_t* const* h_cols, const uint32_t* h_logs, uint32_t n_cols,
-                          DeviceTree& t) {
-    LeafPlan plan = merkle_leaf_plan(h_cols, h_logs, n_cols);
-    DBuf d_tab = upload(c, plan.tab.data(), plan.tab.size());
-    launch_merkle_leaves_dev(c, d_tab.as<LeafColDev>(), plan.segs, n_cols, t);
-}
-
 void launch_merkle_leaves_qm31(Ctx& c, const uint32_t* d_qm31, uint32_t log_size, uint8_t* d_leaves) {
     uint64_t n = 1ull << log_size;
     KTimer kt(c, "merkle_leaves_qm31", 48.0 * (double)n);
@@ -413,8 +350,18 @@ void launch_merkle_leaves_qm31(Ctx& c, const uint32_t* d_qm31, uint32_t log_size
     SR_HIP(hipGetLastError());
 }
 
+// Levels of the parent launch from level k.  A caller that tunes sets their number; the default
+// leaves the top launch at most 2^18 hashes after launches of three levels (445 + 65 + 30 us from
+// 2^24 hashes, 63 + 30 from 2^21, against 591 + 17 and 85 + 17 for launches of ten), four where
+// three would leave 2^19, which takes two more (31 + 15 us for ten levels and the top).
+static uint32_t parent_levels(const Ctx& c, uint32_t k) {
+    if (c.merkle_levels == 10 && k > TREE_TOP_MAX_LOG + 1) return k - 3 == TREE_TOP_MAX_LOG + 1 ? 4 : 3;
+    // at least 8 levels stay for the top launch (up to 2^8 hashes reduce in one workgroup)
+    return std::min(c.merkle_levels, k - 8);
+}
+
 // Wide parent levels (throughput-bound) with merkle_parents_kernel while more than
-// TREE_LAYER_MAX_LOG levels remain, then the top levels and the channel step in one
+// TREE_TOP_MAX_LOG levels remain, then the top levels and the channel step in one
 // tree-layer launch (latency-bound: one quad of lanes per compression on the narrow levels).
 void launch_merkle_parents(Ctx& c, DeviceTree& t, DevChannel* d_ch, uint8_t* d_root_out, uint32_t batch,
                            uint64_t bstride, uint32_t* d_cnt) {
@@ -426,21 +373,29 @@ void launch_merkle_parents(Ctx& c, DeviceTree& t, DevChannel* d_ch, uint8_t* d_r
         else if (d_root_out) SR_HIP(hipMemcpyAsync(d_root_out, t.layers, 32, hipMemcpyDeviceToDevice, c.stream));
         return;
     }
-    while (k > TREE_LAYER_MAX_LOG) {
-        // at least 8 levels stay for the top launch (up to 2^8 hashes reduce in one workgroup)
-        const uint32_t levels = std::min(c.merkle_levels, k - 8);
-        const uint32_t blocks = levels == 1 ? (uint32_t)(((1ull << (k - 1)) + MP_THREADS - 1) / MP_THREADS)
-                                            : (1u << (k - levels));
-        // levels >= 2: 2^(levels-2) threads carry work; at least one wave per block
-        const uint32_t threads = levels == 1 ? MP_THREADS : std::max(64u, 1u << (levels - 2));
+    while (k > TREE_TOP_MAX_LOG) {
+        const uint32_t levels = parent_levels(c, k);
         KTimer kt(c, "merkle_parents L=" + std::to_string(k) + " levels=" + std::to_string(levels),
                   batch * 32.0 * (double)((1ull << k) + (1ull << k) - (1ull << (k - levels))));
-        hipLaunchKernelGGL(merkle_parents_kernel, dim3(blocks, batch), dim3(threads), 0, c.stream, t.layers, k, levels,
-                           c.node_seed, bstride);
+        hipLaunchKernelGGL(merkle_parents_kernel, dim3(1u << (k - 10), batch), dim3(MP_THREADS), 0, c.stream, t.layers,
+                           k, levels, c.node_seed, bstride);
         SR_HIP(hipGetLastError());
         k -= levels;
     }
     launch_tree_top(c, t, k, d_ch, d_root_out, batch, bstride, d_cnt);
+}
+
+// A whole tree from its columns: one launch where the tree-layer kernel can take the leaves
+// (one segment of equal sizes), else leaves, then parents.
+void launch_merkle_tree_dev(Ctx& c, const LeafColDev* d_tab, const std::vector<LeafSeg>& segs, uint32_t n_cols,
+                            DeviceTree& t, uint8_t* d_root_out, uint32_t batch, uint64_t bstride, uint32_t* d_cnt) {
+    if (t.max_log >= 1 && t.max_log <= TREE_COLUMNS_MAX_LOG && segs.size() == 1 && segs[0].ident &&
+        (n_cols + 15) / 16 <= TREE_COLUMNS_MAX_BLOCKS) {
+        launch_tree_from_columns(c, d_tab, n_cols, t, d_root_out, batch, bstride, d_cnt);
+        return;
+    }
+    launch_merkle_leaves_dev(c, d_tab, segs, n_cols, t, batch, bstride);
+    launch_merkle_parents(c, t, nullptr, d_root_out, batch, bstride, d_cnt);
 }
 
 static DeviceTree* new_tree(Ctx& c, uint32_t max_log) {
@@ -477,8 +432,9 @@ DeviceTree* merkle_commit(Ctx& c, const std::vector<const uint32_t*>& cols, cons
         sc[i] = cols[order[i]];
         sl[i] = logs[order[i]];
     }
-    launch_merkle_leaves(c, sc.data(), sl.data(), (uint32_t)sc.size(), *t);
-    launch_merkle_parents(c, *t);
+    LeafPlan plan = merkle_leaf_plan(sc.data(), sl.data(), (uint32_t)sc.size());
+    DBuf d_tab = upload(c, plan.tab.data(), plan.tab.size());
+    launch_merkle_tree_dev(c, d_tab.as<LeafColDev>(), plan.segs, (uint32_t)sc.size(), *t);
     return t;
 }
 

@@ -311,8 +311,7 @@ void plan_commit(Ctx& c, TreeOwner& owner, Committed& out, const std::vector<con
 void launch_commit(Ctx& c, Committed& out, const CommitPlan& cp, uint8_t* d_pack, uint8_t* d_root_out) {
     launch_circle_fft(c, false, (const uint32_t* const*)(d_pack + cp.at_src), (uint32_t* const*)(d_pack + cp.at_dst),
                       cp.n, cp.m, cp.coeff_log);
-    launch_merkle_leaves_dev(c, (const LeafColDev*)(d_pack + cp.at_tab), cp.segs, cp.n, *out.tree);
-    launch_merkle_parents(c, *out.tree, nullptr, d_root_out);
+    launch_merkle_tree_dev(c, (const LeafColDev*)(d_pack + cp.at_tab), cp.segs, cp.n, *out.tree, d_root_out);
 }
 
 void launch_commit_from_evals(Ctx& c, Committed& out, const CommitPlan& cp, uint8_t* d_pack, size_t at_evals,
@@ -326,8 +325,7 @@ void launch_commit_from_evals(Ctx& c, Committed& out, const CommitPlan& cp, uint
         launch_circle_fft(c, true, ev, cf, cp.n, cp.coeff_log, cp.coeff_log);
         launch_circle_fft(c, false, (const uint32_t* const*)cf, ld, cp.n, cp.m, cp.coeff_log);
     }
-    launch_merkle_leaves_dev(c, (const LeafColDev*)(d_pack + cp.at_tab), cp.segs, cp.n, *out.tree);
-    launch_merkle_parents(c, *out.tree, nullptr, d_root_out);
+    launch_merkle_tree_dev(c, (const LeafColDev*)(d_pack + cp.at_tab), cp.segs, cp.n, *out.tree, d_root_out);
 }
 
 void fri_fold_commit_down(Ctx& c, TreeOwner& owner, const uint32_t* d_top, uint32_t top_log, uint32_t last_log,

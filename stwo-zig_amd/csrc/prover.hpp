@@ -230,7 +230,7 @@ void parallel_for(uint32_t n, F&& f) {
 
 // Many wide-Fibonacci proofs of one shape and PCS configuration in single launches
 // (batch_prover.hip): proof k uses prm with trace_seed = seeds[k] (seeds may be NULL: every
-// proof uses prm.trace_seed).  Requires n + log_blowup <= TREE_LAYER_MAX_LOG + 1 and
+// proof uses prm.trace_seed).  Requires n + log_blowup <= 17 and
 // log_last_layer_degree_bound + log_blowup <= FRI_TAIL_MAX_LOG.
 struct BatchStats {
     double device_ms = 0;  // first launch to the readback of the FRI state

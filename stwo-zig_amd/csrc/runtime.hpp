@@ -115,7 +115,7 @@ struct Ctx {
     };
     // Tuning parameters (results are bit-identical for every setting):
     uint32_t fft_tile_log = 13;   // FFT LDS tile, 2^11..2^13 words
-    uint32_t merkle_levels = 10;  // Merkle parent levels per launch, 2..10
+    uint32_t merkle_levels = 10;  // wide Merkle parent levels per launch, 2..9, or 10: see parent_levels
     bool profiling = false;
     std::vector<std::string> profile_only;  // non-empty: record only launches of these classes
     uint32_t profile_every = 1;  // record every k-th launch that matches
@@ -239,15 +239,16 @@ LeafPlan merkle_leaf_plan(const uint32_t* const* h_cols, const uint32_t* h_logs,
 // parents are built.
 void launch_merkle_leaves_dev(Ctx& c, const LeafColDev* d_tab, const std::vector<LeafSeg>& segs, uint32_t n_cols,
                               DeviceTree& t, uint32_t batch = 1, uint64_t bstride = 0);
-// Host arrays in: column device pointers and log sizes, sorted by log size; max log = t.max_log.
-void launch_merkle_leaves(Ctx& c, const uint32_t* const* h_cols, const uint32_t* h_logs, uint32_t n_cols,
-                          DeviceTree& t);
 void launch_merkle_leaves_qm31(Ctx& c, const uint32_t* d_qm31, uint32_t log_size, uint8_t* d_leaves);
 // All parent layers above t's leaves.  With d_ch, the launch reaching the root
 // also mixes it into the device channel and draws the next alpha (root copied to d_root_out).
 // Batches (batch > 1) bring their own completion counters: d_cnt, TREE_CNT_WORDS per proof, zeroed.
 void launch_merkle_parents(Ctx& c, DeviceTree& t, DevChannel* d_ch = nullptr, uint8_t* d_root_out = nullptr,
                            uint32_t batch = 1, uint64_t bstride = 0, uint32_t* d_cnt = nullptr);
+// Leaves and parents (launch_merkle_leaves_dev, then launch_merkle_parents, or one launch).
+void launch_merkle_tree_dev(Ctx& c, const LeafColDev* d_tab, const std::vector<LeafSeg>& segs, uint32_t n_cols,
+                            DeviceTree& t, uint8_t* d_root_out = nullptr, uint32_t batch = 1, uint64_t bstride = 0,
+                            uint32_t* d_cnt = nullptr);
 void launch_merkle_parent_layer(Ctx& c, const uint8_t* d_children, uint32_t log_size, uint8_t* d_parents);
 // FRI folds (folding.zig): line domain halfOdds(log_src) / circle domain CanonicCoset(log_src).
 // d_alpha (optional): read alpha (and alpha^2) from a DevChannel in HBM instead of `alpha`.
@@ -260,19 +261,30 @@ void launch_fold_circle_into_line(Ctx& c, const uint32_t* const* coords, uint32_
 // digest <- H(digest || root); alpha <- drawSecureFelt; root copied to d_root_out (optional).
 void launch_chan_mix_root_draw(Ctx& c, DevChannel* d_ch, const uint8_t* d_root, uint8_t* d_root_out);
 // One tree reduction per launch from level k0 (tree_layer_kernel, kernels_fri.hip), for
-// k0 <= TREE_LAYER_MAX_LOG.  Larger trees (and FRI layers) reduce their wide levels with
-// merkle_parents launches first.  The launches share the context's completion counters,
-// which every launch leaves at zero.
-constexpr uint32_t TREE_LAYER_MAX_LOG = 16;
+// k0 <= TREE_LAYER_MAX_LOG.  The launches share the context's completion counters, which
+// every launch leaves at zero.  Where one launch gives way to wide launches followed by one for
+// the top lies by what the first level's work is (us on one MI355X, one launch / several):
+//   hashes in HBM:      2^17 25 / 11 + 17, 2^18 30 / 12 + 19, 2^19 47 / 31 + 15
+//   rows of columns:    2^17 x 3 29 / 8 + 11 + 17, 2^19 x 16 60 / 22 + 20 + 21; but the 79 blocks of
+//                       1264 columns are better off in the leaf kernels' many waves (a 2^16-instance
+//                       Poseidon proof 1168 / 1069)
+//   a fold, its leaves: 2^18 40 / 14 + 12 + 17; 2^19 no gain
+constexpr uint32_t TREE_LAYER_MAX_LOG = 19;
+constexpr uint32_t TREE_TOP_MAX_LOG = 18;
+constexpr uint32_t TREE_COLUMNS_MAX_LOG = 19;
+constexpr uint32_t TREE_COLUMNS_MAX_BLOCKS = 8;  // 16-word message blocks per leaf
+constexpr uint32_t FRI_LAYER_MAX_LOG = 18;
 constexpr uint32_t TREE_CNT_GROUPS = 16;  // completion sub-counters, then the top counter
 constexpr uint32_t TREE_CNT_STRIDE = 32;  // words between counters (a cache line each)
 constexpr uint32_t TREE_XR_OFFSET = TREE_CNT_STRIDE * (TREE_CNT_GROUPS + 1);  // root exchange after them
-constexpr uint32_t TREE_MAX_BLOCKS = 256;
+constexpr uint32_t TREE_MAX_BLOCKS = 512;
 constexpr uint32_t TREE_CNT_WORDS = TREE_XR_OFFSET + 8 * TREE_MAX_BLOCKS;  // counters + exchange of one tree launch
-enum FriSrc { FRI_SRC_HASHES = 0, FRI_SRC_LINE = 1, FRI_SRC_CIRCLE = 2 };
+enum FriSrc { FRI_SRC_HASHES = 0, FRI_SRC_LINE = 1, FRI_SRC_CIRCLE = 2, FRI_SRC_COLUMNS = 3 };
 struct FriLayerArgs {
     const uint4* src_line;      // FRI_SRC_LINE: the previous line (2^(k0+1) QM31 values)
     const uint32_t* coord[4];   // FRI_SRC_CIRCLE: the 4 coordinate columns (2^(k0+1) words each)
+    const LeafColDev* cols;     // FRI_SRC_COLUMNS: descriptors of n_cols columns of 2^k0 words
+    uint32_t n_cols;
     const uint32_t* inv;        // inverse x (line) or y (circle) of the fold, 2^k0 words
     uint4* dst_line;            // the folded line (2^k0 values)
     uint8_t* tree;              // DeviceTree::layers
@@ -288,6 +300,9 @@ struct FriLayerArgs {
 // Levels k0-1 .. 0 of `t` from its hashes at level k0; with d_ch, the channel step on the root.
 void launch_tree_top(Ctx& c, DeviceTree& t, uint32_t k0, DevChannel* d_ch, uint8_t* d_root_out, uint32_t batch = 1,
                      uint64_t bstride = 0, uint32_t* d_cnt = nullptr);
+// The tree of n_cols columns of 2^t.max_log words each (their leaf hashes, then every level).
+void launch_tree_from_columns(Ctx& c, const LeafColDev* d_tab, uint32_t n_cols, DeviceTree& t, uint8_t* d_root_out,
+                              uint32_t batch = 1, uint64_t bstride = 0, uint32_t* d_cnt = nullptr);
 // One FRI inner layer: fold the line of log_src (or the 4 circle coordinates of log_src) with
 // the alpha in d_ch into d_dst, commit it into `t` (max_log = log_src - 1) and run the channel
 // step on its root (root copied to d_root_out).

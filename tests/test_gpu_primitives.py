@@ -162,6 +162,26 @@ def test_merkle_whole_tree_at_every_split(ctx, log):
         b.free()
 
 
+@pytest.mark.parametrize("n_cols,log", [(16, 1), (17, 2), (33, 4), (128, 5), (129, 5), (31, 9), (128, 11), (129, 11),
+                                        (40, 15), (3, 18), (17, 19), (2, 20), (129, 12)])
+def test_merkle_tree_from_columns_at_its_edges(ctx, n_cols, log):
+    """Equal columns, where leaves and tree are one launch and where they stop being one: full, ragged
+    and several message blocks, leaves by quads and by lanes, the widest and largest shapes of each."""
+    rng = np.random.default_rng(n_cols * 7 + log)
+    cols = rand_cols(rng, n_cols, log)
+    bufs = [ctx.to_device(c) for c in cols]
+    _say("merkle from columns", n_cols, log)
+    tree = ctx.commit_merkle([b.ptr for b in bufs], [log] * n_cols)
+    root, layers = oracle.merkle_commit(cols)
+    assert tree.root == root
+    for lay in range(log + 1):
+        idx = sorted({int(x) for x in rng.integers(0, 1 << lay, size=9)} | {0, (1 << lay) - 1})
+        assert b"".join(tree.read_hashes(lay, idx)) == b"".join(layers[lay][32 * i: 32 * i + 32] for i in idx), lay
+    tree.free()
+    for b in bufs:
+        b.free()
+
+
 @pytest.mark.parametrize("n_cols,log", [(0, 0), (1, 1), (1, 2), (3, 3), (5, 6), (16, 8), (17, 8), (2, 10), (2, 11),
                                         (100, 14), (8, 21)])
 def test_merkle_uniform_matches_oracle(ctx, n_cols, log):
