@@ -176,21 +176,23 @@ struct GdState {
     uint32_t fin[GD_MAX_INST][4][3][4];
     uint32_t rflags[GD_MAX_INST];
 };
-static_assert(sizeof(GdState) % 8 == 0, "state copy in 8-byte words");
+static_assert(sizeof(GdState) % 8 == 0 && sizeof(GdInst) % 8 == 0, "copies in 8-byte words");
 constexpr uint32_t GD_MAX_BX = 1024;   // workgroups per instance in a round launch
 constexpr uint32_t GD_CNT_GROUPS = 16;  // completion sub-counters, one 128-byte line each
 constexpr uint32_t GD_CNT_STRIDE = 32;  // words between counters
 
+// Layers and tables are in device memory (their pointers come from a table, so the compiler is
+// told: a flat access would also wait on LDS).
 __device__ __forceinline__ qm31 gd_ld(const uint32_t* p, uint64_t i) {
-    const uint4 v = ((const uint4*)p)[i];
+    const u32x4 v = ((const SR_GLOBAL u32x4*)p)[i];
     return {{v.x, v.y}, {v.z, v.w}};
 }
 __device__ __forceinline__ void gd_st(uint32_t* p, uint64_t i, qm31 v) {
-    ((uint4*)p)[i] = make_uint4(v.c0.a, v.c0.b, v.c1.a, v.c1.b);
+    ((SR_GLOBAL u32x4*)p)[i] = u32x4{v.c0.a, v.c0.b, v.c1.a, v.c1.b};
 }
 __device__ __forceinline__ qm31 gd_num(uint32_t kind, const uint32_t* num, uint64_t j) {
     if (kind == GKR_LOGUP_GENERIC) return gd_ld(num, j);
-    if (kind == GKR_LOGUP_MULTIPLICITIES) return qfromm(num[j]);
+    if (kind == GKR_LOGUP_MULTIPLICITIES) return qfromm(((gcu32*)num)[j]);
     return qone();
 }
 __device__ __forceinline__ uint32_t gd_fixed_kind(uint32_t kind) {
@@ -244,6 +246,78 @@ __device__ __forceinline__ uint64_t gd_wave_sum8(uint64_t (&x)[8], uint32_t lane
 }
 __device__ __forceinline__ void gd_qstore(uint32_t* w, qm31 v) { qstore(v, w); }
 
+// The channel on one wave (all 64 lanes, every quad computing the same).  Message words go
+// through LDS in lane order (blake2s_quad.hpp): each lane below 24 owns one word and writes
+// it to its place in the 10 rounds.  Lanes 0..15 own the payload words w = 4 (t & 3) + (t >> 2),
+// so that lane t takes word t >> 2 of a QM31 coefficient t & 3; lanes 16..23 own the digest.
+// Boards: mix block 0 (digest || payload 0..7), mix block 1 (payload 8..15 || zeros), draw
+// (digest || counter || zeros).
+constexpr uint32_t GD_CHAN_WORDS = 3 * 160;
+struct GdChan {
+    uint32_t t, ad[10];
+    QuadLane L;
+    uint32_t* bd;
+    uint32_t ilo, ihi;
+    // All threads of the block call it; a barrier must follow.
+    __device__ __forceinline__ GdChan(uint32_t* boards, uint32_t tid) : t(tid), L(tid & 3), bd(boards) {
+        for (uint32_t i = tid; i < GD_CHAN_WORDS; i += blockDim.x) boards[i] = 0;
+        const uint32_t w = t < 16 ? 4 * (t & 3) + (t >> 2) : 0;
+        const uint32_t m = t < 16 ? (w < 8 ? 8 + w : w - 8) : t & 7, blk = t < 16 && w >= 8 ? 160u : 0u;
+#pragma unroll
+        for (int r = 0; r < 10; r++) ad[r] = blk + 16 * r + ((uint32_t)(b2q_places(r) >> (4 * m)) & 15);
+        ilo = L.sel(SR_B2_IV0 ^ 0x01010020u, SR_B2_IV1, SR_B2_IV2, SR_B2_IV3);
+        ihi = L.sel(SR_B2_IV4, SR_B2_IV5, SR_B2_IV6, SR_B2_IV7);
+    }
+    __device__ __forceinline__ uint32_t pay_index() const { return 4 * (t & 3) + (t >> 2); }
+    // This lane's digest word of a hash in the quads (meant in lanes 16..23).
+    __device__ __forceinline__ uint32_t digest_word(uint32_t hlo, uint32_t hhi) const { return (t & 4) ? hhi : hlo; }
+
+    // dv <- Blake2s(digest || payload[0..n_words)), n_words <= 16 and uniform; pv = this lane's
+    // payload word (zero beyond n_words), dv = its digest word.
+    __device__ __forceinline__ void mix(uint32_t& dv, uint32_t pv, uint32_t n_words) const {
+        if (t < 24) {
+            const uint32_t v = t < 16 ? pv : dv;
+#pragma unroll
+            for (int r = 0; r < 10; r++) bd[ad[r]] = v;
+        }
+        qboard_wave_fence();
+        uint32_t hlo = ilo, hhi = ihi;
+        const uint32_t len = 32 + 4 * n_words;
+#pragma unroll 1
+        for (uint32_t b = 0; b < (len > 64 ? 2u : 1u); b++) {
+            const bool last = 64 * (b + 1) >= len;
+            qboard_compress<1>(L, hlo, hhi, bd + 160 * b, 16 * (t & 3), last ? len : 64, last);
+        }
+        dv = digest_word(hlo, hhi);
+    }
+
+    // One secure felt of the digest: words = Blake2s(digest || LE32(n_draws) || 0x00),
+    // n_draws += 1, redrawn until all 8 are < 2p; st = 1 after 64 rejections.
+    __device__ __forceinline__ qm31 draw(uint32_t dv, uint32_t& n_draws, uint32_t& st) const {
+#pragma unroll 1
+        for (uint32_t k = 0; k < 64; k++) {
+            qboard_wave_fence();
+            if (t == 0 || (t >= 16 && t < 24)) {  // lane 0's word is message word 8
+                const uint32_t v = t == 0 ? n_draws : dv;
+#pragma unroll
+                for (int r = 0; r < 10; r++) bd[320 + ad[r]] = v;
+            }
+            qboard_wave_fence();
+            uint32_t olo = ilo, ohi = ihi;
+            qboard_compress<1>(L, olo, ohi, bd + 320, 16 * (t & 3), 37, true);
+            n_draws++;
+            uint32_t bad = (olo >= 2u * P || ohi >= 2u * P) ? 1u : 0u;
+            bad |= quad_perm<QP_ROT1>(bad);
+            bad |= quad_perm<QP_ROT2>(bad);
+            if (!__builtin_amdgcn_readfirstlane(bad))
+                return {{mred64(quad_bcast<0>(olo)), mred64(quad_bcast<1>(olo))},
+                        {mred64(quad_bcast<2>(olo)), mred64(quad_bcast<3>(olo))}};
+        }
+        st = 1;
+        return qzero();
+    }
+};
+
 // Instance view at GKR layer L: active once n_vars + L >= n_layers; its oracle layer has
 // onv + 1 variables, onv = L + n_vars - n_layers.
 struct GdView {
@@ -262,9 +336,12 @@ __device__ __forceinline__ GdView gd_view(const GdInst& in, uint32_t n_layers, u
 // previous layer (2x as long) when `fix`, then the terms at x = 0 and x = 2
 // (gkr_circuit.zig:505-643), each multiplied by eq[k].
 // The term is spread over a quad (all four lanes active, same k): lane j fixes and
-// stores value j, the four values are exchanged with DPP, and every lane forms one
-// product pair f * (A*B + C*D) chosen by its lane index (branch-free); lanes 0 and 2 end
-// with t0 and t2.  Returns e * t in lanes 0 (x = 0) and 2 (x = 2), zero elsewhere.
+// stores value j and, for fractions, forms m_j = n_j + lambda d_j, so that the term
+// (d1 n0 + d0 n1) + lambda d0 d1 is d1 m0 + d0 n1 (at x = 2 the values are 2 v_{2,3} - v_{0,1},
+// and m follows them).  The values are exchanged with DPP, every lane forms one product chosen
+// by its lane index (branch-free) and the pairs add up: a quad's lanes pass through 5 products
+// (6 with lambda as a factor of the sum).  Lanes 0 and 2 end with t0 and t2.
+// Returns e * t in lanes 0 (x = 0) and 2 (x = 2), zero elsewhere.
 __device__ __forceinline__ qm31 gd_term_quad(bool fix, uint32_t kind, const uint32_t* num, const uint32_t* den,
                                              uint32_t* dnum, uint32_t* dden, qm31 r, uint64_t nt, uint64_t k,
                                              qm31 lambda, const uint32_t* eq, uint32_t j) {
@@ -292,15 +369,13 @@ __device__ __forceinline__ qm31 gd_term_quad(bool fix, uint32_t kind, const uint
         const qm31 B = l0 ? d1 : d21;
         x = qmul(A, B);
     } else {
-        const qm31 n0 = quad_bcast_q<0>(n), n1 = quad_bcast_q<1>(n), n2 = quad_bcast_q<2>(n), n3 = quad_bcast_q<3>(n);
-        const qm31 n20 = qsub(qadd(n2, n2), n0), n21 = qsub(qadd(n3, n3), n1);
-        // t0 = (d1 n0 + d0 n1) + lambda d0 d1,  t2 = (d21 n20 + d20 n21) + lambda d20 d21
+        const qm31 m = qadd(n, qmul(d, lambda));
+        const qm31 m0 = quad_bcast_q<0>(m), m2 = quad_bcast_q<2>(m);
+        const qm31 n1 = quad_bcast_q<1>(n), n3 = quad_bcast_q<3>(n);
+        const qm31 m20 = qsub(qadd(m2, m2), m0), n21 = qsub(qadd(n3, n3), n1);
         const qm31 A = l0 ? d1 : (l1 ? d0 : (l2 ? d21 : d20));
-        const qm31 B = l0 ? n0 : (l1 ? d1 : (l2 ? n20 : d21));
-        const qm31 C = l0 ? d0 : (l2 ? d20 : qzero());
-        const qm31 D = l0 ? n1 : n21;
-        x = qadd(qmul(A, B), qmul(C, D));
-        x = qmul((j & 1) ? lambda : qone(), x);
+        const qm31 B = l0 ? m0 : (l1 ? n1 : (l2 ? m20 : n21));
+        x = qmul(A, B);
         x = qadd(x, gd_qperm<QP_ROT1>(x));
     }
     return (l0 || l2) ? qmul(e, x) : qzero();
@@ -391,96 +466,100 @@ __device__ __forceinline__ void gd_round_prep(GdState* S, const GdInst* I, uint3
     gd_qstore(S->fin[i][q][2], C);
 }
 
+// What the end of a round reads of the state, in LDS.
+struct GdFin {
+    uint32_t fin[GD_MAX_INST][4][3][4];
+    uint32_t rflags[GD_MAX_INST];
+    uint32_t alpha_pow[GD_MAX_INST][4];
+    uint32_t sc_claim[GD_MAX_INST][4];
+    uint32_t dg[8];
+};
+
+template <int N>
+__device__ __forceinline__ qm31 gd_row_ror(qm31 v) {
+    const auto f = [](uint32_t x) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x120 + N, 0xF, 0xF, false);
+    };
+    return {{f(v.c0.a), f(v.c0.b)}, {f(v.c1.a), f(v.c1.b)}};
+}
+
 // Turns the round sums (sums[8 i + c]: r(0) then r(2) coordinates before the eq
 // correction, 64-bit) into the batched round polynomial, mixes it and draws the round
 // challenge; the claim update is left pending.  Wave 0 only, with the previous round's
 // update already applied; lane t handles instance t>>2, coefficient t&3.
-__device__ __forceinline__ void gd_finish(GdState* S, const GdInst* I, uint32_t n_inst, uint32_t n_layers, uint32_t L, uint32_t rho,
-                          const unsigned long long* sums, uint32_t* rec) {
+__device__ __forceinline__ void gd_finish(GdState* S, const GdChan& C, const uint32_t (*fin)[4][3][4],
+                                          const uint32_t* rflags, const uint32_t (*alpha_pow)[4],
+                                          const uint32_t (*sc_claim)[4], const uint32_t* dg, uint32_t n_inst,
+                                          uint32_t rho, const unsigned long long* sums, uint32_t* rec) {
     const uint32_t t = threadIdx.x;
     const uint32_t i = t >> 2, q = t & 3;
-    const uint32_t rem = L - rho;
-    (void)I;
-    (void)n_layers;
-    (void)rem;
-    qm31 craw = qzero();
+    uint32_t dv = dg[t & 7];
+    qm31 craw = qzero(), cv = qzero();
     if (i < n_inst) {
-        const uint32_t fl = S->rflags[i];  // set by gd_round_prep for this round
+        const uint32_t fl = rflags[i];  // set by gd_round_prep for this round
         const bool act = fl & 1, part = fl & 2;
+        const qm31 ap = qload(alpha_pow[i]);
         if (part) {
             const unsigned long long* a = sums + 8 * i;
             const qm31 s0 = {{mred64(a[0]), mred64(a[1])}, {mred64(a[2]), mred64(a[3])}};
             const qm31 s2 = {{mred64(a[4]), mred64(a[5])}, {mred64(a[6]), mred64(a[7])}};
-            craw = qadd(qadd(qmul(qload(S->fin[i][q][0]), s0), qmul(qload(S->fin[i][q][2]), s2)),
-                        qload(S->fin[i][q][1]));
+            craw = qadd(qadd(qmul(qload(fin[i][q][0]), s0), qmul(qload(fin[i][q][2]), s2)), qload(fin[i][q][1]));
         } else if (act && q == 0) {
-            craw = qmulm(qload(S->sc_claim[i]), (P + 1) / 2);
+            craw = qmulm(qload(sc_claim[i]), (P + 1) / 2);
         }
-        gd_qstore(S->craw[i][q], craw);
-        if (q == 0) S->pend_flags[i] = fl;
+        cv = qmul(craw, ap);
     }
-    qm31 cv = i < n_inst ? qmul(craw, qload(S->alpha_pow[i])) : qzero();
-#pragma unroll
-    for (int m = 4; m < 32; m <<= 1) cv = qadd(cv, gd_shfl_xor(cv, m));
+    // sum over the instances: lanes 4 and 8 apart within a row of 16, then the two rows
+    cv = qadd(cv, gd_row_ror<8>(cv));
+    cv = qadd(cv, gd_row_ror<4>(cv));
+    if (n_inst > 4) cv = qadd(cv, gd_shfl_xor(cv, 16));
     const uint64_t nzmask = __ballot(t < 4 && !qiszero(cv)) & 0xFull;
     const uint32_t len = nzmask ? 64 - __clzll(nzmask) : 0;
-    if (t < 4) {
-        gd_qstore(rec + 1 + 4 * t, cv);
-        if (t == 0) rec[0] = len;
-        const QuadLane Lq(t);
-        uint32_t dg[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) dg[k] = S->dg[k];
-        uint32_t pay[16];
-        qstore(quad_bcast_q<0>(cv), pay);
-        qstore(quad_bcast_q<1>(cv), pay + 4);
-        qstore(quad_bcast_q<2>(cv), pay + 8);
-        qstore(quad_bcast_q<3>(cv), pay + 12);
-        qchan_mix(Lq, dg, pay, 4 * len);
-        uint32_t nd = 0, st = 0;
-        const qm31 r = qchan_draw(Lq, dg, nd, st);
-        if (t == 0) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) S->dg[k] = dg[k];
-            S->n_draws = nd;
-            if (st) S->status = 1;
-            gd_qstore(S->r, r);
-            gd_qstore(S->asg[rho], r);
-            S->pend = 1;
-            S->pend_rho = rho;
-        }
+    const uint32_t pv = i == 0 ? cv.c0.a : (i == 1 ? cv.c0.b : (i == 2 ? cv.c1.a : cv.c1.b));
+    C.mix(dv, pv, 4 * len);
+    uint32_t nd = 0, st = 0;
+    const qm31 r = C.draw(dv, nd, st);
+    if (t >= 16 && t < 24) S->dg[t & 7] = dv;
+    if (t < 16) rec[1 + C.pay_index()] = pv;
+    if (t == 0) {
+        rec[0] = len;
+        S->n_draws = nd;
+        if (st) S->status = 1;
+        gd_qstore(S->r, r);
+        gd_qstore(S->asg[rho], r);
+        S->pend = 1;
+        S->pend_rho = rho;
+    }
+    if (i < n_inst) {
+        gd_qstore(S->craw[i][q], craw);
+        if (q == 0) S->pend_flags[i] = rflags[i];
     }
 }
 
 // Layer begin (all threads of the block call it; it synchronises the block).
-__device__ __forceinline__ void gd_begin(GdState* S, const GdInst* I, uint32_t n_inst, uint32_t n_layers, uint32_t L) {
+__device__ __forceinline__ void gd_begin(GdState* S, const GdInst* I, const GdChan& C, uint32_t n_inst,
+                                         uint32_t n_layers, uint32_t L) {
     const uint32_t t = threadIdx.x;
     const uint32_t remaining = n_layers - L;
-    if (t < 4) {
-        const QuadLane Lq(t);
-        uint32_t dg[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) dg[k] = S->dg[k];
-        uint32_t nd = S->n_draws, st = 0;
+    if (t < 64) {
+        uint32_t dv = S->dg[t & 7], nd = S->n_draws, st = 0;
         for (uint32_t i = 0; i < n_inst; i++) {
             if (!gd_view(I[i], n_layers, L).active) continue;
-            const uint32_t nc = I[i].kind[0] == GKR_GRAND_PRODUCT ? 1 : 2;
+            const uint32_t nw = I[i].kind[0] == GKR_GRAND_PRODUCT ? 4 : 8;
             const bool fresh = I[i].n_vars == remaining;
-            uint32_t pay[16];
-#pragma unroll
-            for (int k = 0; k < 8; k++) pay[k] = fresh ? (&S->outputs[i][0][0])[k] : (&S->claims[i][0][0])[k];
-#pragma unroll
-            for (int k = 8; k < 16; k++) pay[k] = 0;
-            if (fresh && t == 0)
-                for (int k = 0; k < 8; k++) (&S->claims[i][0][0])[k] = pay[k];
-            qchan_mix(Lq, dg, pay, 4 * nc);
+            const uint32_t w = C.pay_index();
+            uint32_t pv = 0;
+            if (w < 8) {
+                pv = fresh ? (&S->outputs[i][0][0])[w] : (&S->claims[i][0][0])[w];
+                if (fresh && t < 16) (&S->claims[i][0][0])[w] = pv;
+            }
+            C.mix(dv, w < nw ? pv : 0u, nw);
             nd = 0;
         }
-        const qm31 alpha = qchan_draw(Lq, dg, nd, st);
-        const qm31 lambda = qchan_draw(Lq, dg, nd, st);
+        const qm31 alpha = C.draw(dv, nd, st);
+        const qm31 lambda = C.draw(dv, nd, st);
+        if (t >= 16 && t < 24) S->dg[t & 7] = dv;
         if (t == 0) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) S->dg[k] = dg[k];
             S->n_draws = nd;
             if (st) S->status = 1;
             S->pend = 0;
@@ -493,11 +572,15 @@ __device__ __forceinline__ void gd_begin(GdState* S, const GdInst* I, uint32_t n
                 if (a) ap = qmul(ap, alpha);
             }
         }
-    } else if (t >= 64 && t < 64 + L) {
-        // round rho's constants from y = ood[0..L)
+    } else if (t < 128) {
+        // round rho's constants from y = ood[0..L), L < 64; the prefix products by a scan
         const uint32_t rho = t - 64;
-        qm31 pp = qone();
-        for (uint32_t k = 0; k <= rho; k++) pp = qmul(pp, qsub(qone(), qload(S->ood[k])));
+        qm31 pp = rho < L ? qsub(qone(), qload(S->ood[rho])) : qone();
+        for (uint32_t d = 1; d < L; d <<= 1) {
+            const qm31 o = gd_shfl(pp, (int)((t & 63) - d));
+            if (rho >= d) pp = qmul(pp, o);
+        }
+        if (rho < L) {
         const qm31 y = qload(S->ood[rho]);
         const qm31 dd = qsub(qone(), qadd(y, y));
         const qm31 pd = qmul(pp, dd);
@@ -524,6 +607,7 @@ __device__ __forceinline__ void gd_begin(GdState* S, const GdInst* I, uint32_t n
         gd_qstore(pr[9], s1);
         gd_qstore(pr[10], s2);
         if (qiszero(pd) || qiszero(qq)) S->status = 2;
+        }
     }
     __syncthreads();
     if (t < n_inst) {
@@ -553,7 +637,8 @@ __device__ __forceinline__ void gd_eq_entry(const GdState* S, uint32_t L, uint64
 
 // Layer end: masks of every active instance, mixed in order; challenge; next claims and
 // eq point (gkr_prover.zig:232-276, gkr_circuit.zig:341-388).
-__device__ __forceinline__ void gd_end(GdState* S, const GdInst* I, uint32_t n_inst, uint32_t n_layers, uint32_t L, uint32_t* rec_mask) {
+__device__ __forceinline__ void gd_end(GdState* S, const GdInst* I, const GdChan& C, uint32_t n_inst,
+                                       uint32_t n_layers, uint32_t L, uint32_t* rec_mask) {
     const uint32_t t = threadIdx.x;
     if (t < n_inst) {
         const GdView v = gd_view(I[t], n_layers, L);
@@ -599,39 +684,34 @@ __device__ __forceinline__ void gd_end(GdState* S, const GdInst* I, uint32_t n_i
         }
     }
     __syncthreads();
-    if (t < 4) {
-        const QuadLane Lq(t);
-        uint32_t dg[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) dg[k] = S->dg[k];
-        uint32_t nd = S->n_draws, st = 0;
+    if (t < 64) {
+        uint32_t dv = S->dg[t & 7], nd = S->n_draws, st = 0;
         for (uint32_t i = 0; i < n_inst; i++) {
             if (!gd_view(I[i], n_layers, L).active) continue;
             const bool gp = I[i].kind[0] == GKR_GRAND_PRODUCT;
-            uint32_t pay[16];
-#pragma unroll
-            for (int k = 0; k < 16; k++) pay[k] = gp ? (k < 8 ? (&S->mask[i][2][0])[k] : 0u) : (&S->mask[i][0][0])[k];
-            qchan_mix(Lq, dg, pay, gp ? 8 : 16);
+            const uint32_t w = C.pay_index();
+            const uint32_t pv = t < 16 && (!gp || w < 8) ? (&S->mask[i][gp ? 2 : 0][0])[w] : 0u;
+            C.mix(dv, pv, gp ? 8 : 16);
             nd = 0;
         }
-        const qm31 ch = qchan_draw(Lq, dg, nd, st);
+        const qm31 ch = C.draw(dv, nd, st);
+        if (t >= 16 && t < 24) S->dg[t & 7] = dv;
+        // next claims: lane 2 i + c for column c of instance i
+        if (t < 2 * n_inst) {
+            const uint32_t i = t >> 1, c = t & 1;
+            const bool gp = I[i].kind[0] == GKR_GRAND_PRODUCT;
+            if (gd_view(I[i], n_layers, L).active && !(gp && c)) {
+                const uint32_t col = gp ? 1 : c;  // mask column: den (GP) or num, den
+                const qm31 m0 = qload(S->mask[i][2 * col]), m1 = qload(S->mask[i][2 * col + 1]);
+                gd_qstore(S->claims[i][c], qadd(qmul(ch, qsub(m1, m0)), m0));
+            }
+        }
+        if (t < L)
+            for (int k = 0; k < 4; k++) S->ood[t][k] = S->asg[t][k];
         if (t == 0) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) S->dg[k] = dg[k];
             S->n_draws = nd;
             if (st) S->status = 1;
             S->pend = 0;  // the last round's claim update is not needed: the claims come from the masks
-            for (uint32_t i = 0; i < n_inst; i++) {
-                if (!gd_view(I[i], n_layers, L).active) continue;
-                const bool gp = I[i].kind[0] == GKR_GRAND_PRODUCT;
-                for (uint32_t c = 0; c < (gp ? 1u : 2u); c++) {
-                    const uint32_t col = gp ? 1 : c;  // mask column: den (GP) or num, den
-                    const qm31 m0 = qload(S->mask[i][2 * col]), m1 = qload(S->mask[i][2 * col + 1]);
-                    gd_qstore(S->claims[i][c], qadd(qmul(ch, qsub(m1, m0)), m0));
-                }
-            }
-            for (uint32_t j = 0; j < L; j++)
-                for (int k = 0; k < 4; k++) S->ood[j][k] = S->asg[j][k];
             gd_qstore(S->ood[L], ch);
         }
     }
@@ -640,11 +720,13 @@ __device__ __forceinline__ void gd_end(GdState* S, const GdInst* I, uint32_t n_i
 
 // One workgroup: whole layers [L0, L1), the first one starting at round rho0 (its begin
 // already done when rho0 > 0); every layer ends here.  The state lives in LDS meanwhile.
-__global__ __launch_bounds__(GD_FT) void gkr_fused_kernel(GdState* __restrict__ gS, const GdInst* __restrict__ I,
+__global__ __launch_bounds__(GD_FT) void gkr_fused_kernel(GdState* __restrict__ gS, const GdInst* __restrict__ gI,
                                                           uint32_t n_inst, uint32_t n_layers, uint32_t L0, uint32_t L1,
                                                           uint32_t rho0, uint32_t* __restrict__ eq,
                                                           uint32_t* __restrict__ rec) {
     __shared__ GdState S;
+    __shared__ GdInst I[GD_MAX_INST];
+    __shared__ __align__(16) uint32_t boards[GD_CHAN_WORDS];
     // round sums, double-buffered by round parity: the pending-update wave clears the other
     // buffer while a round accumulates into its own (LDS atomics, one add per term and word)
     __shared__ unsigned long long red[2][GD_MAX_INST][8];
@@ -655,7 +737,10 @@ __global__ __launch_bounds__(GD_FT) void gkr_fused_kernel(GdState* __restrict__ 
         uint64_t* dst = (uint64_t*)&S;
         for (uint32_t k = t; k < sizeof(GdState) / 8; k += GD_FT) dst[k] = src[k];
         for (uint32_t k = t; k < 2 * GD_MAX_INST * 8; k += GD_FT) (&red[0][0][0])[k] = 0;
+        const uint64_t* is = (const uint64_t*)gI;
+        for (uint32_t k = t; k < n_inst * (sizeof(GdInst) / 8); k += GD_FT) ((uint64_t*)I)[k] = is[k];
     }
+    const GdChan C(boards, t);
     __syncthreads();
     if (L0 == 0 && rho0 == 0 && t < n_inst) {
         // output layer (gkr_circuit.zig:162-190)
@@ -674,7 +759,7 @@ __global__ __launch_bounds__(GD_FT) void gkr_fused_kernel(GdState* __restrict__ 
     for (uint32_t L = L0; L < L1; L++) {
         const uint32_t rb = L == L0 ? rho0 : 0;
         if (rb == 0) {
-            gd_begin(&S, I, n_inst, n_layers, L);
+            gd_begin(&S, I, C, n_inst, n_layers, L);
             if (L >= 1)
                 for (uint32_t k = t; k < (1u << (L - 1)); k += GD_FT) gd_eq_entry(&S, L, k, eq);
             __syncthreads();
@@ -723,11 +808,11 @@ __global__ __launch_bounds__(GD_FT) void gkr_fused_kernel(GdState* __restrict__ 
             }
             __syncthreads();
             if (t < 64)
-                gd_finish(&S, I, n_inst, n_layers, L, rho, &red[b][0][0],
+                gd_finish(&S, C, S.fin, S.rflags, S.alpha_pow, S.sc_claim, S.dg, n_inst, rho, &red[b][0][0],
                           rec + (uint64_t)(L * (L - 1) / 2 + rho) * GD_REC_ROUND);
             __syncthreads();
         }
-        gd_end(&S, I, n_inst, n_layers, L,
+        gd_end(&S, I, C, n_inst, n_layers, L,
                rec + (uint64_t)total_rounds * GD_REC_ROUND + (uint64_t)L * n_inst * GD_REC_MASK);
     }
     {
@@ -743,7 +828,12 @@ __global__ __launch_bounds__(GD_RT) void gkr_begin_eq_kernel(GdState* __restrict
                                                              uint32_t* __restrict__ eq) {
     const uint64_t k = (uint64_t)blockIdx.x * GD_RT + threadIdx.x;
     if (L >= 1 && k < (1ull << (L - 1))) gd_eq_entry(S, L, k, eq);
-    if (blockIdx.x == 0) gd_begin(S, I, n_inst, n_layers, L);
+    if (blockIdx.x == 0) {
+        __shared__ __align__(16) uint32_t boards[GD_CHAN_WORDS];
+        const GdChan C(boards, threadIdx.x);
+        __syncthreads();
+        gd_begin(S, I, C, n_inst, n_layers, L);
+    }
 }
 
 // One large sum-check round: grid (x: terms, y: instance).  Every workgroup stores its
@@ -758,7 +848,9 @@ __global__ __launch_bounds__(GD_RT) void gkr_round_kernel(GdState* __restrict__ 
                                                           const uint32_t* __restrict__ eq, uint32_t* __restrict__ rec,
                                                           unsigned long long* __restrict__ part, uint32_t* __restrict__ cnt) {
     __shared__ unsigned long long red[GD_RT / 64][8];
-    __shared__ unsigned long long sums[GD_MAX_INST][8];
+    __shared__ unsigned long long sums[GD_MAX_INST][8], rows[GD_MAX_INST][GD_RT / 64][8];
+    __shared__ __align__(16) uint32_t boards[GD_CHAN_WORDS];
+    __shared__ GdFin F;
     __shared__ uint32_t last;
     const uint32_t t = threadIdx.x;
     const uint32_t rem = L - rho;
@@ -828,29 +920,41 @@ __global__ __launch_bounds__(GD_RT) void gkr_round_kernel(GdState* __restrict__ 
     // workgroup's release; this workgroup has nothing of its own to write back
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     if (t <= GD_CNT_GROUPS) atomicExch(&cnt[GD_CNT_STRIDE * t], 0u);
-    for (uint32_t ii = 0, py = 0; ii < n_inst; ii++) {
-        const GdView vi = gd_view(I[ii], n_layers, L);
-        if (!(vi.active && vi.onv >= rem)) continue;
+    // the state the finish reads, and the slots of every summed instance, in one round trip: the
+    // waves share the rows
+    const GdChan C(boards, t);
+    for (uint32_t k = t; k < 48 * n_inst; k += GD_RT) (&F.fin[0][0][0][0])[k] = (&S->fin[0][0][0][0])[k];
+    if (t < 4 * n_inst) {
+        (&F.alpha_pow[0][0])[t] = (&S->alpha_pow[0][0])[t];
+        (&F.sc_claim[0][0])[t] = (&S->sc_claim[0][0])[t];
+    }
+    if (t < n_inst) F.rflags[t] = S->rflags[t];
+    if (t < 8) F.dg[t] = S->dg[t];
+    const uint32_t n_rows = gridDim.y, wpr = n_rows >= 3 ? 1 : (n_rows == 2 ? 2 : 4), wv = t >> 6;
+    for (uint32_t row = wv / wpr; row < n_rows; row += 4 / wpr) {
         uint64_t b8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        const uint32_t row = py++;
-        for (uint32_t x = t; x < gridDim.x; x += GD_RT) {
+        for (uint32_t x = (wv % wpr) * 64 + (t & 63); x < gridDim.x; x += 64 * wpr) {
             unsigned long long* pp = part + ((uint64_t)row * gridDim.x + x) * 8;
 #pragma unroll
             for (int c = 0; c < 8; c++) b8[c] += __hip_atomic_load(&pp[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        {
-            const uint64_t w = gd_wave_sum8(b8, t & 63);
-            if ((t & 7) == 0) red[t >> 6][(t & 63) >> 3] = w;
-        }
-        __syncthreads();
-        if (t < 8) {
-            uint64_t w = 0;
-            for (uint32_t k = 0; k < GD_RT / 64; k++) w += red[k][t];
-            sums[ii][t] = w;
-        }
-        __syncthreads();
+        const uint64_t w = gd_wave_sum8(b8, t & 63);
+        if ((t & 7) == 0) rows[row][wv % wpr][(t & 63) >> 3] = w;
     }
-    if (t < 64) gd_finish(S, I, n_inst, n_layers, L, rho, &sums[0][0], rec + (uint64_t)(L * (L - 1) / 2 + rho) * GD_REC_ROUND);
+    __syncthreads();
+    if (t >= 64) return;
+    if (t < 8 * n_inst) {
+        // instance t / 8 is the row of its rank among the summed ones
+        uint32_t row = 0;
+        for (uint32_t ii = 0; ii < (t >> 3); ii++) row += (F.rflags[ii] >> 1) & 1;
+        uint64_t w = 0;
+        if (F.rflags[t >> 3] & 2)
+            for (uint32_t k = 0; k < wpr; k++) w += rows[row][k][t & 7];
+        sums[t >> 3][t & 7] = w;
+    }
+    qboard_wave_fence();
+    gd_finish(S, C, F.fin, F.rflags, F.alpha_pow, F.sc_claim, F.dg, n_inst, rho, &sums[0][0],
+              rec + (uint64_t)(L * (L - 1) / 2 + rho) * GD_REC_ROUND);
 }
 
 }  // namespace
