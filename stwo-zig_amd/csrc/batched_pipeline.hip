@@ -163,12 +163,15 @@ struct TuningScope {
 void BatchedPipeline::record() {
     TuningScope ts(c, tile_log, levels);
     const uint32_t B = sp.log_blowup;
-    for (auto& sc : classes)
-        launch_circle_fft(c, true, sc.d_eval.as<const uint32_t* const>(), sc.d_coeff.as<uint32_t* const>(), sc.n,
-                          sc.log, sc.log);
-    for (auto& sc : classes)
-        launch_circle_fft(c, false, sc.d_coeff.as<const uint32_t* const>(), sc.d_lde.as<uint32_t* const>(), sc.n,
-                          sc.log + B, sc.log);
+    std::vector<FftGroup> inv, ext;  // largest first
+    for (auto sc = classes.rbegin(); sc != classes.rend(); ++sc) {
+        inv.push_back({sc->d_eval.as<const uint32_t* const>(), sc->d_coeff.as<uint32_t* const>(), sc->n, sc->log,
+                       sc->log});
+        ext.push_back({sc->d_coeff.as<const uint32_t* const>(), sc->d_lde.as<uint32_t* const>(), sc->n, sc->log + B,
+                       sc->log});
+    }
+    launch_circle_fft_groups(c, true, inv);
+    launch_circle_fft_groups(c, false, ext);
     launch_merkle_leaves_dev(c, leaf_tab.as<LeafColDev>(), leaf_segs, sp.n_columns, *tree);
     launch_merkle_parents(c, *tree);
     DevChannel* d_ch = chan.as<DevChannel>();

@@ -31,35 +31,38 @@ void prepare_and_commit(Ctx& c, uint32_t* const* cols, const uint32_t* log_sizes
         max_ext = std::max(max_ext, ext_logs[i]);
     }
     if (max_ext >= 3) c.ensure_tower(max_ext);
-    // one transform launch per distinct log size (the columns of a tree usually share one)
-    std::vector<uint32_t> logs(log_sizes, log_sizes + n_cols);
-    std::sort(logs.begin(), logs.end());
-    logs.erase(std::unique(logs.begin(), logs.end()), logs.end());
-    std::vector<DBuf> tables;
+    // one group of transforms per distinct log size, largest first, over one pointer table
+    std::vector<uint32_t> order(n_cols);
+    for (uint32_t i = 0; i < n_cols; i++) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return log_sizes[x] > log_sizes[y]; });
+    std::vector<uint32_t*> table(2 * (size_t)n_cols);
+    for (uint32_t i = 0; i < n_cols; i++) {
+        table[i] = cols[order[i]];
+        table[n_cols + i] = ext_out[order[i]];
+    }
+    DBuf d_table;
     DeviceTree* t = nullptr;
     double ms = timed(c, [&] {
-        for (uint32_t lg : logs) {
-            std::vector<uint32_t*> src, dst;
-            for (uint32_t i = 0; i < n_cols; i++)
-                if (log_sizes[i] == lg) {
-                    src.push_back(cols[i]);
-                    dst.push_back(ext_out[i]);
-                }
-            tables.push_back(upload(c, src.data(), src.size()));
-            tables.push_back(upload(c, dst.data(), dst.size()));
-            const uint32_t* const* ds = tables[tables.size() - 2].as<const uint32_t* const>();
-            if (interpolate && log_blowup == 1) {
-                // interpolation in place and the extension, fused where the pass plans allow
-                launch_circle_ifft_lde(c, ds, tables[tables.size() - 2].as<uint32_t* const>(),
-                                       tables.back().as<uint32_t* const>(), (uint32_t)src.size(), lg);
-                continue;
+        if (n_cols) d_table = upload(c, table.data(), table.size());
+        uint32_t* const* dt = d_table.as<uint32_t* const>();
+        std::vector<FftGroup> inv, ext;
+        for (uint32_t i = 0; i < n_cols;) {
+            const uint32_t lg = log_sizes[order[i]];
+            uint32_t e = i;
+            while (e < n_cols && log_sizes[order[e]] == lg) e++;
+            const uint32_t* const* ds = (const uint32_t* const*)dt + i;
+            if (interpolate && log_blowup == 1 && (e - i == n_cols || (uint64_t)(e - i) << lg > 1ull << 23)) {
+                // interpolation in place and the extension, fused where the pass plans allow: where
+                // neither would share a launch with another size (one size, or above 1024 tiles)
+                launch_circle_ifft_lde(c, ds, dt + i, dt + n_cols + i, e - i, lg);
+            } else {
+                if (interpolate) inv.push_back({ds, dt + i, e - i, lg, lg});
+                ext.push_back({ds, dt + n_cols + i, e - i, lg + log_blowup, lg});
             }
-            if (interpolate)
-                launch_circle_fft(c, true, ds, tables[tables.size() - 2].as<uint32_t* const>(), (uint32_t)src.size(),
-                                  lg, lg);
-            launch_circle_fft(c, false, ds, tables.back().as<uint32_t* const>(), (uint32_t)src.size(),
-                              lg + log_blowup, lg);
+            i = e;
         }
+        launch_circle_fft_groups(c, true, inv);
+        launch_circle_fft_groups(c, false, ext);
         std::vector<const uint32_t*> ev(ext_out, ext_out + n_cols);
         t = merkle_commit(c, ev, ext_logs);
     });

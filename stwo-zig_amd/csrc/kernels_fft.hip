@@ -19,6 +19,7 @@
 // coalesced C-word segment.  Each element is read from and written to HBM
 // once per pass.
 #include <algorithm>
+#include <vector>
 
 #include "runtime.hpp"
 
@@ -393,20 +394,19 @@ __device__ __forceinline__ void rx_run(uint32_t (&v)[RX], const uint32_t (&w)[4]
     }
 }
 
+// Tile `bid` of a pass, by threads t < 2^(R + LOGC - RX_LOG).
 template <bool INV, int R, int LOGC, bool SP>
-__global__ __launch_bounds__(512) void fft_rx_kernel(const uint32_t* const* __restrict__ src_cols,
-                                                     uint32_t* const* __restrict__ dst_cols,
-                                                     const uint32_t* __restrict__ tower, RxPass ps) {
-    extern __shared__ uint32_t lds[];
+__device__ __forceinline__ void rx_tile(uint32_t* lds, const uint32_t* const* __restrict__ src_cols,
+                                        uint32_t* const* __restrict__ dst_cols, const uint32_t* __restrict__ tower,
+                                        const RxPass& ps, uint32_t bid, uint32_t t) {
     constexpr int TILE_LOG = R + LOGC;
     const uint32_t per_col_log = ps.m - TILE_LOG;
-    const uint32_t col = blockIdx.x >> per_col_log;
-    const uint32_t bb = blockIdx.x & ((1u << per_col_log) - 1);
+    const uint32_t col = bid >> per_col_log;
+    const uint32_t bb = bid & ((1u << per_col_log) - 1);
     const uint32_t lo_blocks_log = ps.s_lo - LOGC;
     const uint32_t lo_blk = bb & ((1u << lo_blocks_log) - 1);
     const uint32_t hi = bb >> lo_blocks_log;
     const uint32_t base = (hi << (ps.s_lo + R)) | (lo_blk << LOGC);
-    const uint32_t t = threadIdx.x;
     const uint32_t lane = t & ((1u << LOGC) - 1);
     const uint32_t r = t >> LOGC;
     uint32_t v[RX];
@@ -415,6 +415,55 @@ __global__ __launch_bounds__(512) void fft_rx_kernel(const uint32_t* const* __re
     rx_group_tw<INV, R, LOGC, S0::B, S0::LO, S0::HI>(w, tower, ps, hi, r, base);
     rx_run<INV, R, LOGC, 0, SP>(v, w, lds, (gcu32*)src_cols[col], (gu32*)dst_cols[col], tower, ps, hi, r, lane, base);
 }
+
+template <bool INV, int R, int LOGC, bool SP>
+__global__ __launch_bounds__(512) void fft_rx_kernel(const uint32_t* const* __restrict__ src_cols,
+                                                     uint32_t* const* __restrict__ dst_cols,
+                                                     const uint32_t* __restrict__ tower, RxPass ps) {
+    extern __shared__ uint32_t lds[];
+    rx_tile<INV, R, LOGC, SP>(lds, src_cols, dst_cols, tower, ps, blockIdx.x, threadIdx.x);
+}
+
+// One pass of several transforms of different sizes: block b takes tile b - first of the group
+// that holds it.  Columns of many sizes come a few to a size, whose own launch leaves most of
+// the chip idle and takes 5..8 us whatever its size.  The threads beyond a smaller tile's leave.
+constexpr uint32_t RX_GROUPS = 16;
+struct RxGroups {
+    struct {
+        const uint32_t* const* src;
+        uint32_t* const* dst;
+        uint32_t first, R, sp, pad;
+        RxPass ps;
+    } g[RX_GROUPS];
+    uint32_t n;
+};
+template <bool INV, bool STRIDED>
+__global__ __launch_bounds__(512) void fft_rx_groups_kernel(const uint32_t* __restrict__ tower, const RxGroups a) {
+    extern __shared__ uint32_t lds[];
+    uint32_t k = 0;
+    while (k + 1 < a.n && blockIdx.x >= a.g[k + 1].first) k++;
+    const uint32_t bid = blockIdx.x - a.g[k].first, t = threadIdx.x, R = a.g[k].R;
+    const RxPass ps = a.g[k].ps;
+    const uint32_t* const* src = a.g[k].src;
+    uint32_t* const* dst = a.g[k].dst;
+    const bool sp = a.g[k].sp;
+    if constexpr (!STRIDED)
+        if (t >= 1u << (R - RX_LOG)) return;
+#define SR_RXG(RR, CC)                                                             \
+    case RR:                                                                       \
+        if (sp) rx_tile<INV, RR, CC, true>(lds, src, dst, tower, ps, bid, t);      \
+        else rx_tile<INV, RR, CC, false>(lds, src, dst, tower, ps, bid, t);        \
+        break;
+    if constexpr (STRIDED) {
+        switch (R) { SR_RXG(4, 9) SR_RXG(5, 8) SR_RXG(6, 7) SR_RXG(7, 6) SR_RXG(8, 5) }
+    } else {
+        switch (R) {
+            SR_RXG(6, 0) SR_RXG(7, 0) SR_RXG(8, 0) SR_RXG(9, 0) SR_RXG(10, 0) SR_RXG(11, 0) SR_RXG(12, 0) SR_RXG(13, 0)
+        }
+    }
+#undef SR_RXG
+}
+
 
 // Interpolation of log n fused with the extension to log n + 1 (blowup 2), over the top
 // strided pass of both transforms (transforms.zig:249-360 then 149-246).  The inverse pass
@@ -761,6 +810,96 @@ void launch_circle_fft(Ctx& c, bool inverse, const uint32_t* const* d_src, uint3
             run_rx_pass(c, true, i == 0 ? d_src : (const uint32_t* const*)d_dst, d_dst, n_cols, passes[i].second,
                         logc_of(passes[i]), ps);
         }
+    }
+}
+
+// Transforms of several sizes (one group each, equal results to a launch_circle_fft per group).
+// A pass of a group with at most RX_GROUP_TILES tiles (four 8192-word tiles per CU and LDS for
+// them: more fill the chip alone, and a launch of its own needs fewer registers) shares its
+// launch with the same-numbered passes of the others; groups of log < 6, and other tiles than
+// 2^13 words, run by themselves.  Extension of 21 columns of 11 sizes 2^9..2^19: 19 launches, 108 us;
+// two, 24 us.
+constexpr uint64_t RX_GROUP_TILES = 1024;
+void launch_circle_fft_groups(Ctx& c, bool inverse, const std::vector<FftGroup>& groups) {
+    struct Step {
+        const FftGroup* g;
+        uint32_t R, logc;
+        bool first;
+        RxPass ps;
+        uint64_t tiles;
+    };
+    uint32_t max_m = 0;
+    for (const FftGroup& g : groups) max_m = std::max(max_m, g.m);
+    if (max_m >= 3) c.ensure_tower(max_m);
+    std::vector<std::vector<Step>> levels;  // passes by position from the contiguous one
+    for (const FftGroup& g : groups) {
+        if (g.n_cols == 0) continue;
+        if (g.m < 6 || c.fft_tile_log != 13) {
+            launch_circle_fft(c, inverse, g.src, g.dst, g.n_cols, g.m, g.src_log);
+            continue;
+        }
+        SR_CHECK(g.m <= 30 && g.src_log <= g.m && (!inverse || g.src_log == g.m), "circle fft: group shape");
+        const auto passes = rx_plan(g.m, 13);
+        for (size_t i = 0; i < passes.size(); i++) {
+            const bool top = i + 1 == passes.size();
+            Step st{&g, passes[i].second, rx_logc(passes[i], 13), inverse ? i == 0 : top, {}, 0};
+            st.ps.m = g.m;
+            st.ps.s_lo = passes[i].first;
+            st.ps.tower_log = c.tower_log;
+            st.ps.src_log = !inverse && top ? g.src_log : g.m;
+            st.ps.dup_top = !inverse && top && g.src_log < g.m;
+            if (inverse && top) rx_set_scale(c, st.ps);
+            st.tiles = (uint64_t)g.n_cols << (g.m - st.R - st.logc);
+            if (levels.size() <= i) levels.resize(i + 1);
+            levels[i].push_back(st);
+        }
+    }
+    for (size_t l = 0; l < levels.size(); l++) {
+        // forward: top passes first.  A group's passes keep their order: each is in a later launch.
+        const size_t li = inverse ? l : levels.size() - 1 - l;
+        const bool strided = li > 0;
+        RxGroups a{};
+        uint64_t blocks = 0;
+        double bytes = 0;
+        const auto flush = [&] {
+            if (!a.n) return;
+            KTimer kt(c, std::string(inverse ? "fft_ifft_groups" : "fft_lde_groups") + (strided ? " strided" : ""),
+                      bytes);
+            const size_t lds = strided ? 4u << 13 : (size_t)((1u << 13) + (1u << 9)) * 4;
+            const uint32_t* tower = inverse ? c.d_itw2 : c.d_tw2;
+            const dim3 grid((uint32_t)blocks), block(512);
+            if (inverse && strided)
+                hipLaunchKernelGGL((fft_rx_groups_kernel<true, true>), grid, block, lds, c.stream, tower, a);
+            else if (inverse)
+                hipLaunchKernelGGL((fft_rx_groups_kernel<true, false>), grid, block, lds, c.stream, tower, a);
+            else if (strided)
+                hipLaunchKernelGGL((fft_rx_groups_kernel<false, true>), grid, block, lds, c.stream, tower, a);
+            else
+                hipLaunchKernelGGL((fft_rx_groups_kernel<false, false>), grid, block, lds, c.stream, tower, a);
+            SR_HIP(hipGetLastError());
+            a = RxGroups{};
+            blocks = 0;
+            bytes = 0;
+        };
+        for (const Step& st : levels[li]) {
+            const FftGroup& g = *st.g;
+            const uint32_t* const* src = st.first ? g.src : (const uint32_t* const*)g.dst;
+            if (st.tiles > RX_GROUP_TILES) {
+                run_rx_pass(c, inverse, src, g.dst, g.n_cols, st.R, st.logc, st.ps);
+                continue;
+            }
+            auto& d = a.g[a.n++];
+            d.src = src;
+            d.dst = g.dst;
+            d.first = (uint32_t)blocks;
+            d.R = st.R;
+            d.sp = inverse ? st.ps.scaled != 0u : st.ps.dup_top != 0u;
+            d.ps = st.ps;
+            blocks += st.tiles;
+            bytes += 4.0 * g.n_cols * ((double)(1ull << st.ps.src_log) + (double)(1ull << g.m));
+            if (a.n == RX_GROUPS) flush();
+        }
+        flush();
     }
 }
 

@@ -206,6 +206,14 @@ struct DBuf {
 // interpolates evaluations of CanonicCoset(m) (src_log == m) and scales by 2^-m.
 void launch_circle_fft(Ctx& c, bool inverse, const uint32_t* const* d_src, uint32_t* const* d_dst, uint32_t n_cols,
                        uint32_t m, uint32_t src_log);
+// Transforms of columns of several sizes: n_cols columns of each group, passes of different groups
+// sharing launches (device pointer tables as above).
+struct FftGroup {
+    const uint32_t* const* src;
+    uint32_t* const* dst;
+    uint32_t n_cols, m, src_log;
+};
+void launch_circle_fft_groups(Ctx& c, bool inverse, const std::vector<FftGroup>& groups);
 // Interpolation of evaluations on CanonicCoset(n) into d_coef (the retained coefficients) and
 // their extension to CanonicCoset(n + 1) into d_lde (device pointer arrays, one entry per
 // column): the top strided passes of the two transforms run as one launch when the pass plans

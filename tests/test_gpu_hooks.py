@@ -93,6 +93,16 @@ def test_prepare_and_commit_owned_and_polys(ctx, logs, blowup):
         x.free()
 
 
+@pytest.mark.parametrize("logs,blowup", [([9, 8, 13, 12, 9, 5, 14, 15, 16, 17, 10, 11, 4, 7, 6], 1),
+                                         ([5, 6, 7, 8, 9, 10, 11, 12, 13], 2), ([19, 18, 17, 16, 15, 3, 2, 1], 3),
+                                         ([1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18], 1),
+                                         ([20, 22, 14], 0), ([21, 6], 1), ([22, 9, 22], 1)])
+def test_prepare_and_commit_of_many_sizes(ctx, logs, blowup):
+    """Columns of different sizes share transform launches: every tile shape and pass count, alone and
+    among others, more sizes than one launch takes, and sizes that keep launches of their own."""
+    test_prepare_and_commit_owned_and_polys(ctx, logs, blowup)
+
+
 def test_prepare_and_commit_without_columns(ctx):
     tree = ctx.prepare_and_commit_owned([], [], 1, [])
     assert tree.root == hashlib.blake2s(b"leaf" + bytes(60)).digest()
