@@ -14,7 +14,7 @@
 //     0, 1, 2, b), so no round inverts anything;
 //   * rounds: fixing the previous round's variable is fused into this round's
 //     sums (in place: index j < h is written by the thread that reads j and
-//     j + h); rounds on layers above 2^GD_SMALL_LOG values are one launch over
+//     j + h); rounds of more than GD_SMALL_TERMS terms are one launch over
 //     many workgroups whose last workgroup (atomic counter, no waiting) turns
 //     the sums into the round polynomial, mixes it and draws the challenge;
 //     smaller rounds, whole small layers and the layer end (masks, challenge,
@@ -134,7 +134,10 @@ namespace {
 
 constexpr uint32_t GD_MAX_INST = 8;
 constexpr uint32_t GD_MAX_VARS = 30;
-constexpr uint32_t GD_SMALL_LOG = 9;  // rounds on layers of <= 2^9 values run in one workgroup (measured best with 10 within 2%)
+// A round of at most this many terms (over its instances) runs in one workgroup: 384 terms take 23K
+// cycles there, 512 25K and 768 36K, a launch over many workgroups 27..29K.
+constexpr uint32_t GD_SMALL_TERMS = 384;
+constexpr uint32_t GD_FUSED_ROUNDS = 55;  // most rounds of one such launch: layers 0..10 of one instance
 constexpr uint32_t GD_FT = 512;       // one-workgroup kernel: 7 summing waves + 1 for the pending update
 constexpr uint32_t GD_RT = 256;       // threads per workgroup of the round and begin kernels
 constexpr uint32_t GD_REC_ROUND = 17;  // [len, 4 QM31] per sum-check round
@@ -163,7 +166,7 @@ struct GdState {
     uint32_t r[4];
     uint32_t ood[GD_MAX_VARS + 1][4];  // eq point of the current layer
     uint32_t asg[GD_MAX_VARS][4];      // challenges of the current layer's rounds
-    uint32_t pre[GD_MAX_VARS][11][4];  // per round: F0, F2, basis rows 1..3 (3 each)
+    uint32_t pre[GD_MAX_VARS][3][4][4];  // per round, for coefficient q: the factors of A, B, C (see fin)
     uint32_t mask[GD_MAX_INST][4][4];
     // the last round's claim update, applied while the next round sums (or dropped at the
     // layer end, where the claims are rebuilt): its coefficients, round and instance flags
@@ -408,62 +411,46 @@ __device__ __forceinline__ GdSrc gd_src(const GdInst& in, uint32_t onv, uint32_t
 // of this round.  With y0 = s0 corr F0, y2 = s2 corr F2 and
 // y1 = claim - y0, the round polynomial's coefficient q of an instance summed in the round is
 // y0 for q = 0 and b1 y0 + b2 y1 + b3 y2 = (b1 - b2) y0 + b2 claim + b3 y2 for q = 1..3 (basis
-// rows b of the round), so A, B, C depend only on values known before the sums.  One full
-// wave; lane t handles instance t>>2, coefficient t&3; the quad's lanes share the instance's
-// claim and correction in registers.
+// rows b of the round), so A, B, C depend only on values known before the sums: the claim times
+// the round's B factor, the correction times its A and C factors (gd_begin).  One full
+// wave; lanes 0..31 take the claims, 32..63 the corrections, lane l of each half instance l>>2,
+// coefficient l&3: four dependent products.
 __device__ __forceinline__ void gd_round_prep(GdState* S, const GdInst* I, uint32_t n_inst, uint32_t n_layers,
                                               uint32_t L, uint32_t rho) {
     const uint32_t t = threadIdx.x & 63;
-    const uint32_t i = t >> 2, q = t & 3;
-    const bool in_range = i < n_inst;
-    qm31 sc = in_range ? qload(S->sc_claim[i]) : qzero();
-    qm31 corr = in_range ? qload(S->corr[i]) : qzero();
+    const uint32_t i = (t & 31) >> 2, q = t & 3;
+    const bool cor = t >= 32, in_range = i < n_inst;
+    // this lane's claim or correction
+    uint32_t* own = cor ? S->corr[in_range ? i : 0] : S->sc_claim[in_range ? i : 0];
+    qm31 val = qload(own);
+    const uint32_t(*pr)[4][4] = S->pre[rho];
+    const qm31 f1 = qload(pr[cor ? 0 : 1][q]), f2 = qload(pr[2][q]);
     if (S->pend) {
         const qm31 r = qload(S->r);
-        const qm31 craw = in_range ? qload(S->craw[i][q]) : qzero();
-        qm31 pw = qone();
-        if (q >= 1) pw = r;
-        if (q >= 2) pw = qmul(pw, r);
-        if (q >= 3) pw = qmul(pw, r);
-        qm31 v = qmul(craw, pw);
-        v = qadd(v, gd_qperm<QP_ROT2>(v));
-        v = qadd(v, gd_qperm<QP_ROT1>(v));  // every lane of the quad: rp_i(r)
+        const qm31 craw = qload(S->craw[in_range ? i : 0][q]), y = qload(S->ood[S->pend_rho]);
         const uint32_t fl = in_range ? S->pend_flags[i] : 0u;
-        if (fl & 1) {
-            sc = v;
-            if (fl & 2) {
-                const qm31 y = qload(S->ood[S->pend_rho]);
-                const qm31 e = qadd(qmul(r, y), qmul(qsub(qone(), r), qsub(qone(), y)));
-                corr = qmul(corr, e);
-            }
-            if (q == 0) {
-                gd_qstore(S->sc_claim[i], sc);
-                if (fl & 2) gd_qstore(S->corr[i], corr);
-            }
+        // claims: c1 r, r^2, c3 r in lanes 1, 2, 3; corrections: r y
+        const qm31 m1 = qmul(cor ? y : (q == 2 ? r : craw), r);
+        // eq(r, y) = r y + (1 - r)(1 - y) = 1 - r - y + 2 r y
+        const qm31 e = qadd(qsub(qsub(qone(), r), y), qadd(m1, m1));
+        // claims: rp(r) = (c0 + c1 r) + (c2 + c3 r) r^2; corrections: corr eq(r, y)
+        const qm31 hi = qadd(quad_bcast_q<2>(craw), quad_bcast_q<3>(m1));
+        const qm31 r2 = quad_bcast_q<2>(m1);
+        const qm31 m2 = qmul(cor ? val : hi, cor ? e : r2);
+        const qm31 lo = qadd(quad_bcast_q<0>(craw), quad_bcast_q<1>(m1));
+        const bool upd = (fl & 1) && (!cor || (fl & 2));
+        if (upd) {
+            val = cor ? m2 : qadd(lo, m2);
+            if (q == 0) gd_qstore(own, val);
         }
     }
     if (!in_range) return;
     const GdView vw = gd_view(I[i], n_layers, L);
     const bool act = vw.active, part = act && vw.onv >= L - rho;
-    if (q == 0) S->rflags[i] = (act ? 1u : 0u) | (part ? 2u : 0u);
+    if (t < 32 && q == 0) S->rflags[i] = (act ? 1u : 0u) | (part ? 2u : 0u);
     if (!part) return;
-    const uint32_t(*pr)[4] = S->pre[rho];
-    const qm31 c0 = qmul(corr, qload(pr[0])), c2 = qmul(corr, qload(pr[1]));
-    qm31 A, B, C;
-    if (q == 0) {
-        A = c0;
-        B = qzero();
-        C = qzero();
-    } else {
-        const uint32_t b = 2 + 3 * (q - 1);
-        const qm31 b1 = qload(pr[b]), b2 = qload(pr[b + 1]), b3 = qload(pr[b + 2]);
-        A = qmul(qsub(b1, b2), c0);
-        B = qmul(b2, sc);
-        C = qmul(b3, c2);
-    }
-    gd_qstore(S->fin[i][q][0], A);
-    gd_qstore(S->fin[i][q][1], B);
-    gd_qstore(S->fin[i][q][2], C);
+    gd_qstore(S->fin[i][q][cor ? 0 : 1], qmul(val, f1));
+    if (cor) gd_qstore(S->fin[i][q][2], qmul(val, f2));
 }
 
 // What the end of a round reads of the state, in LDS.
@@ -572,41 +559,46 @@ __device__ __forceinline__ void gd_begin(GdState* S, const GdInst* I, const GdCh
                 if (a) ap = qmul(ap, alpha);
             }
         }
-    } else if (t < 128) {
-        // round rho's constants from y = ood[0..L), L < 64; the prefix products by a scan
-        const uint32_t rho = t - 64;
+    } else if (t < 256) {
+        // round rho's constants from y = ood[0..L), L < 64: the prefix products by a scan, then wave
+        // q = 1..3 the factors of coefficient q (the first also those of coefficient 0)
+        const uint32_t rho = t & 63, q = t >> 6;
         qm31 pp = rho < L ? qsub(qone(), qload(S->ood[rho])) : qone();
         for (uint32_t d = 1; d < L; d <<= 1) {
-            const qm31 o = gd_shfl(pp, (int)((t & 63) - d));
+            const qm31 o = gd_shfl(pp, (int)(rho - d));
             if (rho >= d) pp = qmul(pp, o);
         }
         if (rho < L) {
-        const qm31 y = qload(S->ood[rho]);
-        const qm31 dd = qsub(qone(), qadd(y, y));
-        const qm31 pd = qmul(pp, dd);
-        const qm31 ipd = qinv(pd);
-        const qm31 ipp = qmul(ipd, dd), idd = qmul(ipd, pp);
-        const qm31 one = qone(), two = qfromm(2), three = qfromm(3);
-        const qm31 b = qmul(qsub(one, y), idd);
-        const qm31 bm1 = qsub(b, one), tmb = qsub(two, b);
-        const qm31 qq = qmul(qmul(b, bm1), tmb);
-        const qm31 iq = qinv(qq);
-        const qm31 ib = qmul(qmul(bm1, tmb), iq), ibm1 = qmul(qmul(b, tmb), iq), itmb = qmul(qmul(b, bm1), iq);
-        const uint32_t inv2 = (P + 1) / 2;
-        const qm31 s0 = qneg(qmulm(ib, inv2)), s1 = ibm1, s2 = qmulm(itmb, inv2);
-        uint32_t(*pr)[4] = S->pre[rho];
-        gd_qstore(pr[0], qmul(qsub(one, y), ipp));                          // F0 = (1-y) / prefix
-        gd_qstore(pr[1], qmul(qsub(qmul(three, y), one), ipp));            // F2 = eq(2, y) / prefix
-        gd_qstore(pr[2], qmul(s0, qadd(two, qmul(three, b))));            // x^1
-        gd_qstore(pr[3], qmul(s1, qadd(b, b)));
-        gd_qstore(pr[4], qmul(s2, b));
-        gd_qstore(pr[5], qneg(qmul(s0, qadd(three, b))));                 // x^2
-        gd_qstore(pr[6], qneg(qmul(s1, qadd(two, b))));
-        gd_qstore(pr[7], qneg(qmul(s2, qadd(one, b))));
-        gd_qstore(pr[8], s0);                                               // x^3
-        gd_qstore(pr[9], s1);
-        gd_qstore(pr[10], s2);
-        if (qiszero(pd) || qiszero(qq)) S->status = 2;
+            const qm31 y = qload(S->ood[rho]);
+            const qm31 dd = qsub(qone(), qadd(y, y));
+            const qm31 pd = qmul(pp, dd);
+            const qm31 ipd = qinv(pd);
+            const qm31 ipp = qmul(ipd, dd), idd = qmul(ipd, pp);
+            const qm31 one = qone(), two = qfromm(2), three = qfromm(3);
+            const qm31 b = qmul(qsub(one, y), idd);
+            const qm31 bm1 = qsub(b, one), tmb = qsub(two, b);
+            const qm31 qq = qmul(qmul(b, bm1), tmb);
+            const qm31 iq = qinv(qq);
+            const qm31 ib = qmul(qmul(bm1, tmb), iq), ibm1 = qmul(qmul(b, tmb), iq), itmb = qmul(qmul(b, bm1), iq);
+            const uint32_t inv2 = (P + 1) / 2;
+            const qm31 s0 = qneg(qmulm(ib, inv2)), s1 = ibm1, s2 = qmulm(itmb, inv2);
+            const qm31 F0 = qmul(qsub(one, y), ipp);                // (1-y) / prefix
+            const qm31 F2 = qmul(qsub(qmul(three, y), one), ipp);  // eq(2, y) / prefix
+            // basis row of x^q: s0 u0, s1 u1, s2 u2
+            qm31 u0 = one, u1 = one, u2 = one;
+            if (q == 1) u0 = qadd(two, qmulm(b, 3)), u1 = qadd(b, b), u2 = b;
+            if (q == 2) u0 = qneg(qadd(three, b)), u1 = qneg(qadd(two, b)), u2 = qneg(qadd(one, b));
+            const qm31 b1 = qmul(s0, u0), b2 = qmul(s1, u1), b3 = qmul(s2, u2);
+            uint32_t(*pr)[4][4] = S->pre[rho];
+            gd_qstore(pr[0][q], qmul(qsub(b1, b2), F0));
+            gd_qstore(pr[1][q], b2);
+            gd_qstore(pr[2][q], qmul(b3, F2));
+            if (q == 1) {
+                gd_qstore(pr[0][0], F0);
+                gd_qstore(pr[1][0], qzero());
+                gd_qstore(pr[2][0], qzero());
+                if (qiszero(pd) || qiszero(qq)) S->status = 2;
+            }
         }
     }
     __syncthreads();
@@ -727,6 +719,9 @@ __global__ __launch_bounds__(GD_FT) void gkr_fused_kernel(GdState* __restrict__ 
     __shared__ GdState S;
     __shared__ GdInst I[GD_MAX_INST];
     __shared__ __align__(16) uint32_t boards[GD_CHAN_WORDS];
+    // round records, written out at the end: a store of the first wave in a round's finish would
+    // hold up its loads of the next round
+    __shared__ uint32_t recs[GD_FUSED_ROUNDS * GD_REC_ROUND];
     // round sums, double-buffered by round parity: the pending-update wave clears the other
     // buffer while a round accumulates into its own (LDS atomics, one add per term and word)
     __shared__ unsigned long long red[2][GD_MAX_INST][8];
@@ -809,13 +804,15 @@ __global__ __launch_bounds__(GD_FT) void gkr_fused_kernel(GdState* __restrict__ 
             __syncthreads();
             if (t < 64)
                 gd_finish(&S, C, S.fin, S.rflags, S.alpha_pow, S.sc_claim, S.dg, n_inst, rho, &red[b][0][0],
-                          rec + (uint64_t)(L * (L - 1) / 2 + rho) * GD_REC_ROUND);
+                          recs + rc * GD_REC_ROUND);
             __syncthreads();
         }
         gd_end(&S, I, C, n_inst, n_layers, L,
                rec + (uint64_t)total_rounds * GD_REC_ROUND + (uint64_t)L * n_inst * GD_REC_MASK);
     }
     {
+        uint32_t* out = rec + (uint64_t)(L0 * (L0 - 1) / 2 + rho0) * GD_REC_ROUND;  // consecutive rounds
+        for (uint32_t k = t; k < rc * GD_REC_ROUND; k += GD_FT) out[k] = recs[k];
         const uint64_t* src = (const uint64_t*)&S;
         uint64_t* dst = (uint64_t*)gS;
         for (uint32_t k = t; k < sizeof(GdState) / 8; k += GD_FT) dst[k] = src[k];
@@ -1051,24 +1048,39 @@ GkrRun* gkr_launch_on_channel(Ctx& c, DevChannel* d_ch, const std::vector<GkrIns
     const GdInst* I = run->d_inst.as<GdInst>();
     uint32_t* eq = run->d_eq.as<uint32_t>();
     uint32_t* rec = run->d_rec.as<uint32_t>();
-    // algorithmic bytes of one sum-check round: 96 B per term (four values read, two fixed
-    // values written, one eq entry) for every instance summed in it
-    auto round_bytes = [&](uint32_t L, uint32_t rho) {
+    // the instances summed in round rho of layer L: active, with onv >= L - rho
+    auto parts = [&](uint32_t L, uint32_t rho) {
         uint32_t n_part = 0;
         for (uint32_t k = 0; k < n_inst; k++)
             n_part += inst[k].n_vars + L >= n_layers && inst[k].n_vars + L - n_layers >= L - rho;
-        return 96.0 * (double)(1ull << (L - rho - 1)) * n_part;
+        return n_part;
     };
+    // algorithmic bytes of one sum-check round: 96 B per term (four values read, two fixed
+    // values written, one eq entry) for every instance summed in it
+    auto round_bytes = [&](uint32_t L, uint32_t rho) {
+        return 96.0 * (double)(1ull << (L - rho - 1)) * parts(L, rho);
+    };
+    // first round of layer L from which every round is a one-workgroup one
+    auto first_small = [&](uint32_t L) {
+        uint32_t rho = L;
+        while (rho > 0 && ((uint64_t)parts(L, rho - 1) << (L - rho)) <= GD_SMALL_TERMS) rho--;
+        return rho;
+    };
+    uint32_t n_small = 0;  // layers below run whole in one workgroup
+    while (n_small < n_layers && first_small(n_small) == 0) n_small++;
+    SR_CHECK(n_small * (n_small ? n_small - 1 : 0) / 2 <= GD_FUSED_ROUNDS, "gkr: rounds of one launch");
     {
         double bytes = 0;
-        for (uint32_t L = 1; L < std::min(n_layers, GD_SMALL_LOG); L++)
+        for (uint32_t L = 1; L < n_small; L++)
             for (uint32_t rho = 0; rho < L; rho++) bytes += round_bytes(L, rho);
         KTimer kt(c, "gkr_small_layers", bytes);
-        hipLaunchKernelGGL(gkr_fused_kernel, dim3(1), dim3(GD_FT), 0, c.stream, S, I, n_inst, n_layers, 0u,
-                           std::min(n_layers, GD_SMALL_LOG), 0u, eq, rec);
+        hipLaunchKernelGGL(gkr_fused_kernel, dim3(1), dim3(GD_FT), 0, c.stream, S, I, n_inst, n_layers, 0u, n_small, 0u,
+                           eq, rec);
         SR_HIP(hipGetLastError());
     }
-    for (uint32_t L = GD_SMALL_LOG; L < n_layers; L++) {
+    for (uint32_t L = n_small; L < n_layers; L++) {
+        const uint32_t small = first_small(L);  // > 0: a layer's first round is its largest
+        SR_CHECK(small > 0 && L - small <= GD_FUSED_ROUNDS, "gkr: rounds of one launch");
         {
             KTimer kt(c, "gkr_begin_eq", 16.0 * (double)(1ull << (L - 1)));
             const uint64_t blocks = ((1ull << (L - 1)) + GD_RT - 1) / GD_RT;
@@ -1076,24 +1088,20 @@ GkrRun* gkr_launch_on_channel(Ctx& c, DevChannel* d_ch, const std::vector<GkrIns
                                n_layers, L, eq);
             SR_HIP(hipGetLastError());
         }
-        uint32_t rho = 0;
-        for (; L - rho >= GD_SMALL_LOG; rho++) {
+        for (uint32_t rho = 0; rho < small; rho++) {
             const uint64_t nt = 1ull << (L - rho - 1);
             // summing workgroups per instance, plus one column for the round-start prep
             const uint64_t bx = std::min<uint64_t>((nt + GD_RT / 4 - 1) / (GD_RT / 4), GD_MAX_BX - 1) + 1;
-            uint32_t n_part = 0;  // instances summed in this round: active with onv >= L - rho
-            for (uint32_t k = 0; k < n_inst; k++)
-                n_part += inst[k].n_vars + L >= n_layers && inst[k].n_vars + L - n_layers >= L - rho;
             KTimer kt(c, "gkr_round", round_bytes(L, rho));
-            hipLaunchKernelGGL(gkr_round_kernel, dim3((uint32_t)bx, n_part), dim3(GD_RT), 0, c.stream, S, I, n_inst,
-                               n_layers, L, rho, (const uint32_t*)eq, rec, run->d_part.as<unsigned long long>(),
-                               run->d_cnt.as<uint32_t>());
+            hipLaunchKernelGGL(gkr_round_kernel, dim3((uint32_t)bx, parts(L, rho)), dim3(GD_RT), 0, c.stream, S, I,
+                               n_inst, n_layers, L, rho, (const uint32_t*)eq, rec,
+                               run->d_part.as<unsigned long long>(), run->d_cnt.as<uint32_t>());
             SR_HIP(hipGetLastError());
         }
         double bytes = 0;
-        for (uint32_t r2 = rho; r2 < L; r2++) bytes += round_bytes(L, r2);
+        for (uint32_t r2 = small; r2 < L; r2++) bytes += round_bytes(L, r2);
         KTimer kt(c, "gkr_small_rounds", bytes);
-        hipLaunchKernelGGL(gkr_fused_kernel, dim3(1), dim3(GD_FT), 0, c.stream, S, I, n_inst, n_layers, L, L + 1, rho,
+        hipLaunchKernelGGL(gkr_fused_kernel, dim3(1), dim3(GD_FT), 0, c.stream, S, I, n_inst, n_layers, L, L + 1, small,
                            eq, rec);
         SR_HIP(hipGetLastError());
     }
