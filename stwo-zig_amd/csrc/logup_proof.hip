@@ -227,7 +227,6 @@ void prove_logup_xor(Ctx& c, uint32_t log_n, uint64_t seed, const ProveParams& p
             }
             DBuf ds = upload(c, src.data(), 12), dd = upload(c, dst.data(), 12);
             launch_circle_fft(c, false, ds.as<const uint32_t* const>(), dd.as<uint32_t* const>(), 12, n + 1, n);
-            c.sync();
         }
         DBuf dev = upload(c, ev.data(), 12);
         KTimer kt(c, "logup_composition", 4.0 * 13 * (double)CN + 16.0 * (double)CN);
@@ -237,7 +236,6 @@ void prove_logup_xor(Ctx& c, uint32_t log_n, uint64_t seed, const ProveParams& p
         SR_HIP(hipGetLastError());
         DBuf dcc = upload(c, cc, 4);
         launch_circle_fft(c, true, dcc.as<const uint32_t* const>(), dcc.as<uint32_t* const>(), 4, n + 1, n + 1);
-        c.sync();
     }
     {
         std::vector<const uint32_t*> halves(8);
@@ -264,26 +262,30 @@ void prove_logup_xor(Ctx& c, uint32_t log_n, uint64_t seed, const ProveParams& p
     std::vector<const uint32_t*> all_cf;
     for (auto* T : trees) all_cf.insert(all_cf.end(), T->coeffs.begin(), T->coeffs.end());
     const uint32_t NC = (uint32_t)all_cf.size();  // 20
-    auto eval_at = [&](const SamplePoint& p, const std::vector<const uint32_t*>& cols) {
-        qm31 f[32];
-        f[0] = p.y;
-        f[1] = p.x;
-        for (uint32_t k = 2; k < n; k++) {
-            const qm31 sq = qsqr(f[k - 1]);
-            f[k] = qsub(qadd(sq, sq), qone());
-        }
-        DBuf w(&c, N * 16), o(&c, 16 * cols.size());
-        launch_eval_weights(c, f, n, w.as<uint32_t>());
-        DBuf dcol = upload(c, cols.data(), cols.size());
-        launch_eval_columns(c, dcol.as<const uint32_t* const>(), (uint32_t)cols.size(), n, w.as<uint32_t>(),
-                            o.as<uint32_t>());
-        std::vector<uint32_t> h(4 * cols.size());
-        SR_HIP(hipMemcpyAsync(h.data(), o.p, 16 * cols.size(), hipMemcpyDeviceToHost, c.stream));
+    // both points' values in one readback
+    std::vector<uint32_t> cur(4 * NC), prv(4 * t2.coeffs.size());
+    {
+        DBuf w(&c, N * 16), o(&c, 4 * (cur.size() + prv.size()));
+        const auto eval_at = [&](const SamplePoint& p, const std::vector<const uint32_t*>& cols, uint32_t* out) {
+            qm31 f[32];
+            f[0] = p.y;
+            f[1] = p.x;
+            for (uint32_t k = 2; k < n; k++) {
+                const qm31 sq = qsqr(f[k - 1]);
+                f[k] = qsub(qadd(sq, sq), qone());
+            }
+            launch_eval_weights(c, f, n, w.as<uint32_t>());
+            DBuf dcol = upload(c, cols.data(), cols.size());
+            launch_eval_columns(c, dcol.as<const uint32_t* const>(), (uint32_t)cols.size(), n, w.as<uint32_t>(), out);
+        };
+        eval_at(oods, all_cf, o.as<uint32_t>());
+        eval_at(prev, t2.coeffs, o.as<uint32_t>() + cur.size());
+        uint32_t* h = (uint32_t*)c.pinned(4 * (cur.size() + prv.size()));
+        SR_HIP(hipMemcpyAsync(h, o.p, 4 * (cur.size() + prv.size()), hipMemcpyDeviceToHost, c.stream));
         c.sync();
-        return h;
-    };
-    const std::vector<uint32_t> cur = eval_at(oods, all_cf);
-    const std::vector<uint32_t> prv = eval_at(prev, t2.coeffs);
+        memcpy(cur.data(), h, 4 * cur.size());
+        memcpy(prv.data(), h + cur.size(), 4 * prv.size());
+    }
     // tree/column/sample order: the interaction columns carry (current, previous)
     std::vector<uint32_t> sv;
     std::vector<uint32_t> n_samples;
