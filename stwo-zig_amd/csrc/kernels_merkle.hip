@@ -360,6 +360,11 @@ static uint32_t parent_levels(const Ctx& c, uint32_t k) {
     return std::min(c.merkle_levels, k - 8);
 }
 
+// A batch whose hashes at level k fill the device several times over (8 blocks of a parent launch
+// per CU): its trees are bound by instructions like one large tree, and half of a tree launch's time
+// goes to levels that keep one wave of a workgroup busy.
+static bool wide_batch(uint32_t batch, uint32_t k) { return batch > 1 && k >= 11 && ((uint64_t)batch << k) >= 1ull << 21; }
+
 // Wide parent levels (throughput-bound) with merkle_parents_kernel while more than
 // TREE_TOP_MAX_LOG levels remain, then the top levels and the channel step in one
 // tree-layer launch (latency-bound: one quad of lanes per compression on the narrow levels).
@@ -373,8 +378,8 @@ void launch_merkle_parents(Ctx& c, DeviceTree& t, DevChannel* d_ch, uint8_t* d_r
         else if (d_root_out) SR_HIP(hipMemcpyAsync(d_root_out, t.layers, 32, hipMemcpyDeviceToDevice, c.stream));
         return;
     }
-    while (k > TREE_TOP_MAX_LOG) {
-        const uint32_t levels = parent_levels(c, k);
+    while (k > TREE_TOP_MAX_LOG || wide_batch(batch, k)) {
+        const uint32_t levels = wide_batch(batch, k) ? 3 : parent_levels(c, k);
         KTimer kt(c, "merkle_parents L=" + std::to_string(k) + " levels=" + std::to_string(levels),
                   batch * 32.0 * (double)((1ull << k) + (1ull << k) - (1ull << (k - levels))));
         hipLaunchKernelGGL(merkle_parents_kernel, dim3(1u << (k - 10), batch), dim3(MP_THREADS), 0, c.stream, t.layers,
@@ -390,7 +395,7 @@ void launch_merkle_parents(Ctx& c, DeviceTree& t, DevChannel* d_ch, uint8_t* d_r
 void launch_merkle_tree_dev(Ctx& c, const LeafColDev* d_tab, const std::vector<LeafSeg>& segs, uint32_t n_cols,
                             DeviceTree& t, uint8_t* d_root_out, uint32_t batch, uint64_t bstride, uint32_t* d_cnt) {
     if (t.max_log >= 1 && t.max_log <= TREE_COLUMNS_MAX_LOG && segs.size() == 1 && segs[0].ident &&
-        (n_cols + 15) / 16 <= TREE_COLUMNS_MAX_BLOCKS) {
+        (n_cols + 15) / 16 <= TREE_COLUMNS_MAX_BLOCKS && !wide_batch(batch, t.max_log)) {
         launch_tree_from_columns(c, d_tab, n_cols, t, d_root_out, batch, bstride, d_cnt);
         return;
     }

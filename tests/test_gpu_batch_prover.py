@@ -59,6 +59,18 @@ def test_batch_equals_one_proof_path(ctx, n, w, seeds, pcs):
         sv.verify_proof(proofs[k], "wide_fibonacci", {"log_n_rows": n, "sequence_len": w}, pcs)
 
 
+@pytest.mark.parametrize("n,w,K", [(10, 3, 1024), (10, 3, 1023), (13, 17, 128), (14, 5, 66)])
+def test_wide_batch_equals_one_proof_path(ctx, n, w, K):
+    """Batches around the size from which the trees' wide levels have launches of their own."""
+    print("wide batch %dx%d K=%d" % (n, w, K), flush=True)
+    pcs = dict(pow_bits=4, log_blowup_factor=1, log_last_layer_degree_bound=0, n_queries=3)
+    seeds = [1000 + 7 * k for k in range(K)]
+    proofs, _ = ctx.prove_wide_fibonacci_batch(n, w, seeds=seeds, trace_mode=1, **pcs)
+    for k in sorted({0, 1, K // 2, K - 2, K - 1}):
+        one, _ = ctx.prove_wide_fibonacci(n, w, trace_mode=1, trace_seed=seeds[k], stats=False, **pcs)
+        assert proofs[k] == one, "proof %d differs from the one-proof path" % k
+
+
 def test_batch_reference_trace_is_the_golden_proof(ctx):
     idx = json.load(open(os.path.join(GOLD, "wide_fibonacci_goldens.json")))
     e = idx["wide_fibonacci_log10_seq8_pow10"]
