@@ -473,7 +473,8 @@ typedef struct {
 } stwo_rocm_batched_spec;
 int stwo_rocm_batched_create(stwo_rocm_ctx* ctx, const stwo_rocm_batched_spec* spec, stwo_rocm_batched** out);
 /* Launch-shape tuning (results are bit-identical for every setting): FFT LDS tile 2^11..2^13 words,
- * Merkle parent levels per launch 2..10.  Applies to this pipeline only (the context's other work
+ * Merkle parent levels per launch 2..10 (10, the default, leaves the trees above 2^19 hashes to the
+ * library: launches of three levels).  Applies to this pipeline only (the context's other work
  * keeps its shapes) and recaptures the graph.  A replay recaptures by itself when the context's
  * twiddle tower has moved since the capture (a larger transform on the context, twiddles_prepare,
  * release_cached). */

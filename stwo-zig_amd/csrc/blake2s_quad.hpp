@@ -12,8 +12,8 @@
 // part of it.  From 16 words in registers every lane selects its 2 words of a half round (6
 // selects; fewer where words are constant zeros).  From LDS in lane order (QuadIo below) a
 // round's 4 words are one 16-byte read: about 300 instructions for a compression and its
-// exchange against 420 and an exchange of plain words.  FRI layers of 2^16 / 2^11 values went
-// from 30 / 22 to 26.5 / 18.3 us, the one-workgroup tail from 107 to 97 us (2^16-row XOR proof).
+// exchange against 420 and an exchange of plain words.  With it FRI layers of 2^15 / 2^11 values
+// went from 30 / 22 to 26.5 / 18.3 us, the one-workgroup tail from 107 to 97 us (2^16-row XOR proof).
 // All four lanes of a quad must be active together.
 #pragma once
 #include "blake2s.hpp"
