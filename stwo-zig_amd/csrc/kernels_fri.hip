@@ -299,7 +299,7 @@ __device__ __forceinline__ TrChan tr_chan_init(const TrQuad& Q, uint32_t* chan, 
 }
 
 // Channel step on a root held by every quad of the first wave, which runs it, as (rlo, rhi)
-// (MerkleChannel.mixRoot then drawSecureFelt, as chan_mix_root_draw_quad).
+// (MerkleChannel.mixRoot then drawSecureFelt, as chan_mix_root_draw_thread).
 __device__ __forceinline__ void tr_chan_step(const TrQuad& Q, uint32_t* chan, uint32_t rlo, uint32_t rhi, TrChan& C,
                                              DevChannel* __restrict__ ch) {
     const QuadLane& L = Q.L;
