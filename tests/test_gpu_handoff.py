@@ -14,7 +14,7 @@ import pytest
 import oracle
 import stark_verifier as sv
 from test_gpu_hooks import _commit_layers_restated, _m31
-from test_gpu_logup import _proof_case, dev
+from test_gpu_logup import ROW_CASES, _proof_case, assert_wide_rounds, dev, row_case
 
 pytestmark = pytest.mark.gpu
 
@@ -70,13 +70,11 @@ def test_fri_cascade_long_run(ctx):
 
 
 def test_gkr_batch_long_run(ctx):
-    """A batch whose first layers run over many workgroups (2^10 and 2^9 values), proven again
-    and again with a one-workgroup batch in between."""
-    insts = _proof_case(ctx, "mixed_big")
-    small = _proof_case(ctx, "mixed")
+    """A batch whose large rounds run over many workgroups and sum two to eight instances, proven again and
+    again with a one-workgroup batch and one of one to four summed instances in between."""
+    insts, joining, small = row_case("rows_8"), row_case("joining"), _proof_case(ctx, "mixed")
     digest = bytes(range(32, 64))
-    ref = oracle.gkr_prove(insts, digest)
-    ref_small = oracle.gkr_prove(small, digest)
+    ref, ref_joining, ref_small = (oracle.gkr_prove(x, digest) for x in (insts, joining, small))
     keep = []
 
     def on_device(cases):
@@ -88,13 +86,19 @@ def test_gkr_batch_long_run(ctx):
             out.append((kind, dn, dd, nv))
         return out
 
-    d_insts, d_small = on_device(insts), on_device(small)
+    d_insts, d_joining, d_small = on_device(insts), on_device(joining), on_device(small)
     try:
+        for name, cases, d, r in (("rows_8", insts, d_insts, ref), ("joining", joining, d_joining, ref_joining)):
+            words = assert_wide_rounds(ctx, [nv for _, _, _, nv in cases], ROW_CASES[name][1],
+                                       lambda: ctx.gkr_prove_batch(d, digest))
+            assert np.array_equal(words, r), name
         for run in range(GKR_RUNS):
             words = ctx.gkr_prove_batch(d_insts, digest)
             assert np.array_equal(words, ref), "GKR run %d differs" % run
             if run % 2 == 0:
                 assert np.array_equal(ctx.gkr_prove_batch(d_small, digest), ref_small)
+            if run % 3 == 0:
+                assert np.array_equal(ctx.gkr_prove_batch(d_joining, digest), ref_joining), "after run %d" % run
             if run % 50 == 0:
                 _say("gkr run", run)
     finally:

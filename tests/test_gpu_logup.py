@@ -185,7 +185,7 @@ def _proof_case(ctx, shape):
                                  "mixed_big": 7, "eight": 8, "one_var": 9, "edge8": 10, "edge9": 11}[shape])
     if shape == "gp":
         return [(0, None, rand_q(rng, 32), 5)]
-    if shape == "gp_big":  # rounds above 2^8 values run over many workgroups
+    if shape == "gp_big":  # its first round (512 terms) runs over many workgroups
         return [(0, None, rand_q(rng, 1 << 11), 11)]
     if shape == "mixed_big":
         return [(1, rand_q(rng, 1 << 10), rand_q(rng, 1 << 10), 10), (0, None, rand_q(rng, 1 << 9), 9),
@@ -199,7 +199,7 @@ def _proof_case(ctx, shape):
         return out
     if shape == "one_var":
         return [(1, rand_q(rng, 2), rand_q(rng, 2), 1)]
-    if shape in ("edge8", "edge9"):  # around the one-workgroup threshold
+    if shape in ("edge8", "edge9"):  # two instances, rounds of up to 128 and 256 terms: all in one workgroup
         nv = 8 if shape == "edge8" else 9
         return [(1, rand_q(rng, 1 << nv), rand_q(rng, 1 << nv), nv), (3, None, rand_q(rng, 1 << nv), nv)]
     if shape == "generic":
@@ -239,6 +239,79 @@ def _locate(words, n_layers, idx):
                 return "layer %d mask of instance %d word %d" % (layer, int(words[p]), idx - p)
             p += 2 + 8 * nc
     return "tail (outputs, ood, claims, digest) word %d" % (idx - p)
+
+
+# Batches by (kind, variables) with rounds over many workgroups, and the numbers of instances summed in those
+# rounds (rows of the launch's partial sums): one, two and from three on are reduced differently at a round's end.
+ROW_CASES = {
+    "at_384": ([(1, 9), (2, 9), (3, 9)], set()),  # the largest round has 384 terms: one workgroup
+    "at_512": ([(1, 9), (2, 9), (3, 9), (0, 9)], {4}),
+    "rows_1": ([(1, 12)], {1}),
+    "rows_2": ([(3, 12), (2, 12)], {2}),
+    "rows_3": ([(2, 12), (0, 12), (1, 12)], {3}),
+    "rows_5": ([(1, 11), (0, 11), (3, 11), (2, 11), (1, 11)], {5}),
+    "joining": ([(2, 11), (1, 13), (3, 10), (0, 12)], {1, 2, 3, 4}),  # the deepest not first
+    "rows_8": ([(1, 9), (2, 12), (0, 8), (3, 11), (1, 10), (0, 12), (2, 9), (3, 8)], {2, 3, 4, 6, 8}),
+    # layer 9: 256 terms in the first round, 1024 in the second
+    "small_first": ([(0, 9), (1, 10), (2, 9), (3, 9), (1, 9), (0, 9), (2, 9), (3, 9)], {1, 8}),
+}
+
+
+def row_case(name):
+    rng = np.random.default_rng(1000 + sorted(ROW_CASES).index(name))
+    out = []
+    for kind, nv in ROW_CASES[name][0]:
+        num = rand_q(rng, 1 << nv) if kind == 1 else rand_m(rng, 1 << nv, 1000) if kind == 2 else None
+        out.append((kind, num, rand_q(rng, 1 << nv), nv))
+    return out
+
+
+def wide_rounds(n_vars, small_terms=384):
+    """(layer, round, instances summed) of every round over many workgroups: those of a layer up to its last
+    one with more than small_terms terms.  Instance k is summed in round rho when n_vars[k] + rho >= max."""
+    n_layers = max(n_vars)
+    out = []
+    for layer in range(n_layers):
+        rows = [sum(nv + layer >= n_layers and nv + rho >= n_layers for nv in n_vars) for rho in range(layer)]
+        wide = [rho for rho in range(layer) if rows[rho] << (layer - rho - 1) > small_terms]
+        out += [(layer, rho, rows[rho]) for rho in range(max(wide) + 1)] if wide else []
+    return out
+
+
+def assert_wide_rounds(ctx, n_vars, rows, prove):
+    """`prove` runs a batch of n_vars variables once: it launches the many-workgroup round kernel for exactly
+    the rounds that the rule gives it, and those sum the stated numbers of instances."""
+    rounds = wide_rounds(n_vars)
+    assert {r for _, _, r in rounds} == rows
+    ctx.profile_enable(True)
+    try:
+        words = prove()
+        classes = ctx.profile_read()
+    finally:
+        ctx.profile_enable(False)
+    assert classes.get("gkr_round", {"launches": 0})["launches"] == len(rounds), sorted(classes)
+    return words
+
+
+@pytest.mark.parametrize("name", list(ROW_CASES))
+def test_gkr_prove_batch_over_many_workgroups(ctx, name):
+    """Rounds over many workgroups that sum 1..8 instances of every kind, joined by shallower instances, at
+    the number of terms from which they are launched; the launches are counted."""
+    _say("gkr rows", name)
+    insts = row_case(name)
+    digest = bytes(range(64, 96))
+    keep, dinst = [], []
+    for kind, num, den, nv in insts:
+        dn, dd = dev(ctx, num) if num is not None else None, dev(ctx, den)
+        keep += [dn, dd]
+        dinst.append((kind, dn, dd, nv))
+    n_vars = [nv for _, _, _, nv in insts]
+    words = assert_wide_rounds(ctx, n_vars, ROW_CASES[name][1], lambda: ctx.gkr_prove_batch(dinst, digest))
+    ref = oracle.gkr_prove(insts, digest)
+    assert words.size == ref.size
+    diff = np.nonzero(words != ref)[0]
+    where = _locate(ref, max(n_vars), int(diff[0])) if diff.size else ""
+    assert diff.size == 0, "first difference at word %d: %s" % (int(diff[0]), where)
 
 
 @pytest.mark.parametrize("shape", ["gp", "generic", "mixed", "one_var", "edge8", "edge9", "gp_big", "mixed_big",
