@@ -75,7 +75,7 @@ constexpr uint64_t b2q_places(int r) {
 // needs (two wait states) and the compiler would otherwise fill with s_nop, since it puts the
 // addition that a permuted operand's partner comes from right before it: 1360 cycles a
 // compression instead of 1040.  All permuted rows are written inside the block, so nothing
-// that the compiler puts before it matters.
+// that the compiler puts before it matters.  The rows are early-clobber: x is read after a is written.
 #define SR_B2Q_STEP(PA, PC, PD)                                                    \
     asm("v_add3_u32 %0, %0, %1, %4\n\t"                                            \
         "v_xor_b32_e32 %3, %3, %0\n\t"                                             \
@@ -90,7 +90,7 @@ constexpr uint64_t b2q_places(int r) {
         "v_add_u32_dpp %2, %2, %3 quad_perm:" PC " row_mask:0xf bank_mask:0xf\n\t" \
         "v_xor_b32_e32 %1, %1, %2\n\t"                                             \
         "v_alignbit_b32 %1, %1, %1, 12"                                            \
-        : "+v"(a), "+v"(b), "+v"(c), "+v"(d)                                       \
+        : "+&v"(a), "+&v"(b), "+&v"(c), "+&v"(d)                                   \
         : "v"(y), "v"(x), "s"(0x01000302u), "s"(0x00030201u))
 
 // (hlo, hhi) = chaining words (q, 4+q) in and out; msg(r) = this lane's words of round r in
