@@ -134,10 +134,21 @@ namespace {
 
 constexpr uint32_t GD_MAX_INST = 8;
 constexpr uint32_t GD_MAX_VARS = 30;
-// A round of at most this many terms (over its instances) runs in one workgroup: 384 terms take 23K
-// cycles there, 512 25K and 768 36K, a launch over many workgroups 27..29K.
+// A round of at most this many terms (over its instances) runs in one workgroup.  By itself a round
+// of 384 terms takes 23K cycles there, 512 25K and 768 36K, and a launch over many workgroups
+// 27..29K.  Whole proofs are flat up to 512 (us at limits of 256 / 384 / 512 / 768, runs of one side
+// differ by 5..50): one instance of 2^18 1507 / 1499 / 1492 / 1491, two of 2^18 and 2^16 1641 / 1643 /
+// 1654 / 1650, four of 2^16 1551 / 1542 / 1567 / 1561, four of 2^18, 2^17, 2^15, 2^9 1824 / 1815 / 1810 /
+// 1874.  So the limit is the middle one, the best or within 1% on each.
 constexpr uint32_t GD_SMALL_TERMS = 384;
-constexpr uint32_t GD_FUSED_ROUNDS = 55;  // most rounds of one such launch: layers 0..10 of one instance
+// Most rounds of one such launch: layers 0..9 of one instance (layer L has L rounds, the first of 2^(L-1)
+// terms).
+constexpr uint32_t gd_fused_rounds(uint32_t terms) {
+    uint32_t top = 0;
+    while ((1u << top) <= terms) top++;
+    return top * (top + 1) / 2;
+}
+constexpr uint32_t GD_FUSED_ROUNDS = gd_fused_rounds(GD_SMALL_TERMS);
 constexpr uint32_t GD_FT = 512;       // one-workgroup kernel: 7 summing waves + 1 for the pending update
 constexpr uint32_t GD_RT = 256;       // threads per workgroup of the round and begin kernels
 constexpr uint32_t GD_REC_ROUND = 17;  // [len, 4 QM31] per sum-check round
@@ -1079,7 +1090,9 @@ GkrRun* gkr_launch_on_channel(Ctx& c, DevChannel* d_ch, const std::vector<GkrIns
         SR_HIP(hipGetLastError());
     }
     for (uint32_t L = n_small; L < n_layers; L++) {
-        const uint32_t small = first_small(L);  // > 0: a layer's first round is its largest
+        // > 0: the instances of a round depend on rho alone, so its terms double from one layer to the next,
+        // and a layer after the first one with a large round has one too
+        const uint32_t small = first_small(L);
         SR_CHECK(small > 0 && L - small <= GD_FUSED_ROUNDS, "gkr: rounds of one launch");
         {
             KTimer kt(c, "gkr_begin_eq", 16.0 * (double)(1ull << (L - 1)));
