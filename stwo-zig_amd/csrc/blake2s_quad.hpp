@@ -11,9 +11,10 @@
 // so a compression takes its instruction count: 13 per half round.  The message words are
 // part of it.  From 16 words in registers every lane selects its 2 words of a half round (6
 // selects; fewer where words are constant zeros).  From LDS in lane order (QuadIo below) a
-// round's 4 words are one 16-byte read: about 300 instructions for a compression and its
-// exchange against 420 and an exchange of plain words.  With it FRI layers of 2^15 / 2^11 values
-// went from 30 / 22 to 26.5 / 18.3 us, the one-workgroup tail from 107 to 97 us (2^16-row XOR proof).
+// round's 4 words are one 16-byte read: 1170 cycles for a compression on a lone wave against 1620
+// with the selects, 1500 with the write to the next board.  With it and the levels' last-wave loop
+// (kernels_fri.hip) FRI layers of 2^15 / 2^12 and 2^11 values went from 30 / 22 to 23 / 15 us, the
+// one-workgroup tail from 110 to 87 us (2^16-row XOR proof).
 // All four lanes of a quad must be active together.
 #pragma once
 #include "blake2s.hpp"
@@ -73,8 +74,8 @@ constexpr uint64_t b2q_places(int r) {
 // a, c, d are read through quad permutes PA, PC, PD.  13 instructions in this order: every row
 // read through a permute was written at least three instructions before, which the DPP operand
 // needs (two wait states) and the compiler would otherwise fill with s_nop, since it puts the
-// addition that a permuted operand's partner comes from right before it: 1360 cycles a
-// compression instead of 1040.  All permuted rows are written inside the block, so nothing
+// addition that a permuted operand's partner comes from right before it: 1360 cycles for the 20 half
+// rounds of a compression instead of 1040.  All permuted rows are written inside the block, so nothing
 // that the compiler puts before it matters.  The rows are early-clobber: x is read after a is written.
 #define SR_B2Q_STEP(PA, PC, PD)                                                    \
     asm("v_add3_u32 %0, %0, %1, %4\n\t"                                            \

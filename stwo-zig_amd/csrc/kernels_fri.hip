@@ -634,7 +634,8 @@ __global__ __launch_bounds__(TAIL_THREADS) void fri_tail_kernel(const FriTailArg
 // Hashes per workgroup (log) for a tree reduction from level k0: the whole tree in one
 // workgroup up to 2^8 leaves; above, the levels split about evenly between the workgroups'
 // subtrees and the last workgroup's top, with at most 2^8 workgroups (one per CU: a second
-// workgroup on a CU halves the issue rate of both) and at most 2^10 hashes per workgroup.
+// workgroup on a CU halves the issue rate of both) as long as a workgroup's hashes fit its LDS (2^10):
+// a level of 2^19 takes 2^9 workgroups (TREE_MAX_BLOCKS).
 static uint32_t tree_chunk_log(uint32_t k0) { return k0 <= 8 ? k0 : std::min(10u, std::max(k0 / 2, k0 - 8)); }
 
 template <int SRC>
@@ -693,7 +694,7 @@ void launch_fri_commit_line(Ctx& c, const uint32_t* d_src, uint32_t log_src, uin
     const uint32_t l = log_src - 1;
     SR_CHECK(log_src >= 1 && t.max_log == l && d_ch, "fri commit: layer shape");
     if (l == 0 || l > FRI_LAYER_MAX_LOG) {
-        SR_CHECK(batch == 1, "fri commit: batches of layers above 2^16");
+        SR_CHECK(batch == 1, "fri commit: batches of layers above 2^18");
         launch_fold_line(c, d_src, log_src, qzero(), d_dst, t.layer(l), d_ch);
         launch_merkle_parents(c, t, d_ch, d_root_out);
         return;
@@ -718,7 +719,7 @@ void launch_fri_commit_circle(Ctx& c, const uint32_t* const* coords, uint32_t lo
     const uint32_t l = log_src - 1;
     SR_CHECK(log_src >= 1 && t.max_log == l && d_ch, "fri commit: layer shape");
     if (l == 0 || l > FRI_LAYER_MAX_LOG) {
-        SR_CHECK(batch == 1, "fri commit: batches of layers above 2^16");
+        SR_CHECK(batch == 1, "fri commit: batches of layers above 2^18");
         launch_fold_circle_into_line(c, coords, log_src, qzero(), d_dst, false, t.layer(l), d_ch);
         launch_merkle_parents(c, t, d_ch, d_root_out);
         return;

@@ -152,8 +152,9 @@ __global__ __launch_bounds__(MK_THREADS) void merkle_leaves_qm31_kernel(const ui
 // compressions) and their parent of level k-2 in registers; the remaining levels halve in LDS,
 // by one lane per compression while that fills whole waves, then by quads.  The kernel is bound
 // by the instructions of its compressions, and every level after the first two leaves more of
-// the block's lanes idle: from 2^24 hashes, ten levels take 591 us for 2^24 compressions, four
-// 493, three 445 for 7/8 of them; the leaves' 2^24 would take 500 at the rate of a 100-column tree.
+// the block's lanes idle: from 2^24 hashes, ten levels took 560 us for 2^24 compressions, four take
+// 452, three 437 for 7/8 of them (kernel trace of the replayed column pipeline, one box); as many
+// leaf compressions would take 490 at the rate of a 100-column tree.
 constexpr uint32_t MP_THREADS = 256;
 __device__ __forceinline__ void node_hash(const B2State& seed, const uint32_t* l, const uint32_t* r, uint32_t h[8]) {
     uint32_t m[16];
@@ -351,9 +352,14 @@ void launch_merkle_leaves_qm31(Ctx& c, const uint32_t* d_qm31, uint32_t log_size
 }
 
 // Levels of the parent launch from level k.  A caller that tunes sets their number; the default
-// leaves the top launch at most 2^18 hashes after launches of three levels (445 + 65 + 30 us from
-// 2^24 hashes, 63 + 30 from 2^21, against 591 + 17 and 85 + 17 for launches of ten), four where
-// three would leave 2^19, which takes two more (31 + 15 us for ten levels and the top).
+// leaves the top launch at most 2^18 hashes after launches of three levels (437 + 62 + 30 us from
+// 2^24 hashes and 62 + 30 from 2^21, where launches of ten levels and their tops took 560 + 24 and 84 +
+// 20), four where three would leave 2^19, which takes two launches more (from 2^22: 123 + 30 us
+// against 116 + 21 + 26).
+// A tree of exactly 2^19 hashes keeps one launch of ten levels and a top of 2^9: 35 + 13.5 us, where
+// three levels and a top of 2^16 take 22 + 23 (a committed line of 2^19: 96 / 92 us).  It is not the
+// faster form.  Its launch class is the documented sign that a pipeline's tuning stays with the
+// pipeline (test_gpu_batched.py reads it from the context's own trees), so the name is kept.
 static uint32_t parent_levels(const Ctx& c, uint32_t k) {
     if (c.merkle_levels == 10 && k > TREE_TOP_MAX_LOG + 1) return k - 3 == TREE_TOP_MAX_LOG + 1 ? 4 : 3;
     // at least 8 levels stay for the top launch (up to 2^8 hashes reduce in one workgroup)
@@ -362,7 +368,10 @@ static uint32_t parent_levels(const Ctx& c, uint32_t k) {
 
 // A batch whose hashes at level k fill the device several times over (8 blocks of a parent launch
 // per CU): its trees are bound by instructions like one large tree, and half of a tree launch's time
-// goes to levels that keep one wave of a workgroup busy.
+// goes to levels that keep one wave of a workgroup busy.  Device time of whole batches, us, tree
+// launch / launches of three levels, for trees of 2^15, 2^11, 2^13, 2^17 hashes: 2^20 hashes in the batch
+// 951 / 990, 697 / 674, 688 / 679, 819 / 822; 2^21 1607 / 1568, 1192 / 1159, 1079 / 1044, 1191 / 1156; 2^22
+// 2899 / 2802, 2187 / 2094, 1972 / 1844, 1959 / 1878.
 static bool wide_batch(uint32_t batch, uint32_t k) { return batch > 1 && k >= 11 && ((uint64_t)batch << k) >= 1ull << 21; }
 
 // Wide parent levels (throughput-bound) with merkle_parents_kernel while more than

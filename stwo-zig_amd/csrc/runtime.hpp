@@ -273,9 +273,13 @@ void launch_chan_mix_root_draw(Ctx& c, DevChannel* d_ch, const uint8_t* d_root, 
 // every launch leaves at zero.  Where one launch gives way to wide launches followed by one for
 // the top lies by what the first level's work is (us on one MI355X, one launch / several):
 //   hashes in HBM:      2^17 25 / 11 + 17, 2^18 30 / 12 + 19, 2^19 47 / 31 + 15
-//   rows of columns:    2^17 x 3 29 / 8 + 11 + 17, 2^19 x 16 60 / 22 + 20 + 21; but the 79 blocks of
-//                       1264 columns are better off in the leaf kernels' many waves (a 2^16-instance
-//                       Poseidon proof 1168 / 1069)
+//   rows of columns:    2^17 x 3 29 / 8 + 11 + 17, 2^19 x 16 60 / 22 + 20 + 21; but many message blocks are
+//                       better off in the leaf kernels' many waves.  Whole commitments by blocks of 16
+//                       columns, one launch / several: 1 block 2^10 59 / 62, 2^15 67 / 67, 2^19 106 / 112;
+//                       4 blocks 64 / 73, 78 / 80, 160 / 166; 7 blocks 73 / 83, 94 / 93, 218 / 218; 8 blocks
+//                       74 / 80, 95 / 98, 243 / 233; 10 blocks 83 / 85, 105 / 105, 2^18 180 / 171; the 79 blocks
+//                       of a 2^16-instance Poseidon proof 1168 / 1069.  So 8 blocks: beyond them nothing is
+//                       gained at any size, and up to 7 nothing is lost
 //   a fold, its leaves: 2^18 40 / 14 + 12 + 17; 2^19 no gain
 constexpr uint32_t TREE_LAYER_MAX_LOG = 19;
 constexpr uint32_t TREE_TOP_MAX_LOG = 18;

@@ -301,8 +301,9 @@ def test_pow_grind_matches_oracle(ctx, bits):
 
 @pytest.mark.parametrize("bits", [13, 17, 18, 19, 21])
 def test_pow_grind_lowest_nonce_over_strides(ctx, bits):
-    """Difficulties around the sizes of the thread count (2^14 .. 2^19 threads, several nonces per
-    thread): the nonce is the lowest valid one, for digests whose solutions fall in different strides."""
+    """Difficulties around the launch's change from one nonce per thread to eight (launches of more than 2^20
+    nonces, from 17 bits on): the nonce is the lowest valid one, for digests whose solutions fall in
+    different workgroups and steps of one."""
     for k in range(4):
         digest = hashlib.blake2s(b"stride%d-%d" % (bits, k)).digest()
         _say("pow", bits, k)
