@@ -849,6 +849,10 @@ void launch_circle_fft_groups(Ctx& c, bool inverse, const std::vector<FftGroup>&
             st.ps.src_log = !inverse && top ? g.src_log : g.m;
             st.ps.dup_top = !inverse && top && g.src_log < g.m;
             if (inverse && top) rx_set_scale(c, st.ps);
+            // the shapes fft_rx_groups_kernel has (it leaves a tile of any other as it is)
+            SR_CHECK(i == 0 ? st.logc == 0 && st.R >= 6 && st.R <= 13
+                            : st.logc == 13 - st.R && st.R >= 4 && st.R <= 8,
+                     "fft groups: no kernel for pass shape R=" + std::to_string(st.R));
             st.tiles = (uint64_t)g.n_cols << (g.m - st.R - st.logc);
             if (levels.size() <= i) levels.resize(i + 1);
             levels[i].push_back(st);
